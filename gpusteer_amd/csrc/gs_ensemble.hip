@@ -31,7 +31,7 @@
 #include <vector>
 
 #include "gs_ensemble.hpp"
-#include "gs_knn_core.hpp"
+#include "gs_knn_team.hpp"
 
 namespace gs {
 
@@ -156,7 +156,8 @@ __global__ __launch_bounds__(kBlock, PART == 0 ? 5 : 1) void e_knn(
     const float* __restrict__ wmy, const float* __restrict__ wmz, const float* __restrict__ ox,
     const float* __restrict__ oy, const float* __restrict__ oz) {
     GS_FLAT_LDS
-    const uint32_t blk = PART == 0 ? xcd_block(blockIdx.x, gridDim.x) : blocks[xcd_block(blockIdx.x, gridDim.x)];
+    uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    if (blocks) blk = blocks[blk];
     const uint32_t s = blk * blockDim.x + threadIdx.x;
     const EnsPop& P = E.pops[E.block_pop[blk]];
     // Padding lanes stay through the searches (the wavefront completes its
@@ -210,6 +211,75 @@ __global__ __launch_bounds__(kBlock, PART == 0 ? 5 : 1) void e_knn(
             brute_small<8>(h, q.x, q.y, q.z, n, x, y, z);
             store_local<8>(h, kk, N, s, o, out.out_map);
         }
+    };
+    small(S.k_walls, S.nw, wmx + S.w0, wmy + S.w0, wmz + S.w0, out.walls);
+    small(S.k_obs, S.no, ox + S.o0, oy + S.o0, oz + S.o0, out.obs);
+}
+
+// e_knn with G lanes per query (gs_knn_team.hpp): a block of kBlock slots
+// becomes G thread blocks of kBlock / G queries.
+template <int G, int PART>
+__global__ __launch_bounds__(kBlock) void e_knn_team(
+    EnsDev E, const uint32_t* __restrict__ blocks, uint32_t N, uint32_t k, const float4* __restrict__ spos,
+    const uint32_t* __restrict__ start, const uint32_t* __restrict__ new_to_old,
+    const uint32_t* __restrict__ old_to_new, EnsKnnOut out, const float* __restrict__ wmx,
+    const float* __restrict__ wmy, const float* __restrict__ wmz, const float* __restrict__ ox,
+    const float* __restrict__ oy, const float* __restrict__ oz) {
+    __shared__ TeamLds<G, 8, 1> lds;
+    TeamList<G, 8, 1> L(lds, k);
+    const uint32_t id = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t blk = blocks ? blocks[id / G] : id / G;
+    const uint32_t s = blk * kBlock + (id % G) * (kBlock / G) + threadIdx.x / G;
+    const EnsPop& P = E.pops[E.block_pop[blk]];
+    const bool active = s < P.a0 + P.n;
+    const float4 q = active ? spos[s] : make_float4(0.f, 0.f, 0.f, 0.f);
+    // The list to column `row` (mapped: rows and neighbour values through
+    // out_map, as store_idx; otherwise rows only, as store_local).
+    auto store = [&](uint32_t* __restrict__ o, bool mapped) {
+        if (!active) return;
+        const uint32_t row = out.out_map ? out.out_map[s] : s;
+        for (uint32_t j = L.lane; j < L.k; j += G) {
+            uint32_t v = (int)j < L.cnt ? L.best_slot[j] : UINT32_MAX;
+            if (mapped && out.out_map && v != UINT32_MAX) v = out.out_map[v];
+            o[(size_t)j * N + row] = v;
+        }
+    };
+    if constexpr (PART == 0) {
+        float thr = INFINITY;
+        if (out.seed_self)
+            thr = team_seed_bound(L, active, out.seed_self, N, active ? new_to_old[s] : 0u, N, old_to_new, q.x, q.y,
+                                  q.z, spos);
+        const FlatQuery Q{q.x, q.y, q.z, thr, s, active};
+        knn_search_team(L, Q, P.g, N, spos, start + P.c0);
+        store(out.self, true);
+        return;
+    }
+    if (P.kind != GS_SCENARIO_CHOKE) return;
+    const EnsPop& O = E.pops[P.other];
+    if (O.n > 0) {
+        const float cap2 = E.scens[P.scen].other_cap2;
+        float thr = cap2;
+        if (out.seed_other)
+            thr = fminf(cap2, team_seed_bound(L, active, out.seed_other, N, active ? new_to_old[s] : 0u, N, old_to_new,
+                                              q.x, q.y, q.z, spos));
+        if (active && box_beyond(out.box + 6 * (size_t)P.other, q.x, q.y, q.z, cap2)) thr = -1.f;
+        const FlatQuery Q{q.x, q.y, q.z, thr, UINT32_MAX, active};
+        knn_search_team(L, Q, O.g, N, spos, start + O.c0);
+    }
+    store(out.other, true);
+    const EnsScen& S = E.scens[P.scen];
+    auto small = [&](uint32_t kk, uint32_t n, const float* x, const float* y, const float* z, uint32_t* o) {
+        team_fence();  // the stores above read the list that is reset here
+        L.k = kk;
+        L.cnt = 0;
+        L.lim = INFINITY;
+        for (uint32_t j0 = 0; j0 < n; j0 += G) {
+            const uint32_t j = j0 + L.lane;
+            const float d2 = j < n ? sqdist(q.x, q.y, q.z, x[j], y[j], z[j]) : NAN;
+            L.add(d2 <= L.lim, d2, j, j);
+        }
+        L.reduce();
+        store(o, false);
     };
     small(S.k_walls, S.nw, wmx + S.w0, wmy + S.w0, wmz + S.w0, out.walls);
     small(S.k_obs, S.no, ox + S.o0, oy + S.o0, oz + S.o0, out.obs);
@@ -584,27 +654,59 @@ static EnsDev ens_dev(gs_ensemble_s* e) {
     return EnsDev{e->d_pops.p, e->d_scens.p, e->d_block_pop.p};
 }
 
+// The searches of every agent's own group (all blocks), then the crowds'
+// other lists: one lane per query (7-entry lists for k = 7) or teams.
+struct EnsSearch {
+    EnsDev E;
+    uint32_t N, k;
+    const float4* spos;
+    const uint32_t *start, *new_to_old, *old_to_new;
+    EnsKnnOut out;
+    const float *wmx, *wmy, *wmz, *ox, *oy, *oz;
+};
+template <int PART>
+static void launch_search(const EnsSearch& a, int lanes, const uint32_t* blocks, size_t nblocks, hipStream_t st) {
+    if (nblocks == 0) return;
+    const unsigned nb = (unsigned)nblocks;
+#define GS_ES(KERNEL, COUNT)                                                                                          \
+    KERNEL<<<COUNT, kBlock, 0, st>>>(a.E, blocks, a.N, a.k, a.spos, a.start, a.new_to_old, a.old_to_new, a.out, a.wmx, \
+                                     a.wmy, a.wmz, a.ox, a.oy, a.oz)
+    if (lanes == 16) GS_ES((e_knn_team<16, PART>), nb * 16);
+    else if (lanes == 8) GS_ES((e_knn_team<8, PART>), nb * 8);
+    else if (a.k == 7) GS_ES((e_knn<7, PART>), nb);
+    else GS_ES((e_knn<8, PART>), nb);
+#undef GS_ES
+    GS_LAUNCHED("e_knn");
+}
+static void ens_search(gs_ensemble_s* e, const EnsKnnOut& out, int lanes, hipStream_t st) {
+    const EnsSearch a{ens_dev(e),   e->N,           e->k,           e->spos.p,     e->start.p,
+                      e->new_to_old.p, e->old_to_new.p, out,             e->walls[9].p, e->walls[10].p,
+                      e->walls[11].p, e->obs[0].p,     e->obs[1].p,     e->obs[2].p};
+    launch_search<0>(a, lanes, nullptr, e->N / kBlock, st);
+    launch_search<1>(a, lanes, e->d_blocks_choke.p, e->blocks_choke.size(), st);
+}
+// Lanes per query of a step's searches.  Crowds press together at the gap and
+// at their goals; one lane per query then leaves the step waiting for the few
+// wavefronts whose queries scan thousands of agents of a cell each, so teams
+// pay up to larger sizes than for a flock: 24 scenarios of 220,000 agents over
+// 400 steps 1.03 - 1.19 -> 0.36 ms per step; 64 scenarios of 384,000 agents 0.22 ->
+// 0.27 ms while they are spread out and 0.69 -> 0.35 after 160 steps (left
+// with one lane: the first steps would be slower).
+constexpr uint32_t kTeamMaxCrowds = 262144;
+static int step_lanes(const gs_ensemble_s* e) {
+    const int lanes = team_lanes(e->N, e->k);
+    return lanes == 1 && !e->blocks_choke.empty() && e->N <= kTeamMaxCrowds ? 8 : lanes;
+}
+// Of a calibration's searches: its crowds stay near their uniform start.
+// Forward pass of 50 steps, one lane / 8 lanes: 16,384 agents 4.9 / 3.5 ms,
+// 65,536 5.3 / 4.8, 131,072 6.3 / 6.7.
+constexpr uint32_t kTeamMaxCalib = 98304;
+
 // Exact KNN lists of every agent (own group, other group capped, walls,
 // obstacles) for state held in a fixed order: the positions px/py/pz are
 // binned into a sorted snapshot (the ensemble's bin buffers as scratch; its
 // own state and KNN containers are not touched) and the lists are written in
 // the fixed order (rows and neighbour values are fixed indices).  Seeds are
-// The ensemble search kernels for the ensemble's k (7-entry lists for
-// k = 7): own groups over all blocks, then the crowds' other lists.
-#define GS_E_KNN(...)                                                                            \
-    do {                                                                                         \
-        if (e->k == 7)                                                                           \
-            e_knn<7, 0><<<nblocks, kBlock, 0, st>>>(E, nullptr, __VA_ARGS__);                    \
-        else                                                                                     \
-            e_knn<8, 0><<<nblocks, kBlock, 0, st>>>(E, nullptr, __VA_ARGS__);                    \
-        GS_LAUNCHED("e_knn");                                                                    \
-        const unsigned ncb = (unsigned)e->blocks_choke.size();                                   \
-        if (ncb && e->k == 7)                                                                    \
-            e_knn<7, 1><<<ncb, kBlock, 0, st>>>(E, e->d_blocks_choke.p, __VA_ARGS__);            \
-        else if (ncb)                                                                            \
-            e_knn<8, 1><<<ncb, kBlock, 0, st>>>(E, e->d_blocks_choke.p, __VA_ARGS__);            \
-    } while (0)
-
 // previous lists in the same fixed order (or NULL).
 void ens_search_fixed(gs_ensemble_s* e, float* px, float* py, float* pz, const uint32_t* ids_fixed,
                       uint32_t* ids_scratch, float* const scratch[3], const uint32_t* seed_self,
@@ -637,10 +739,7 @@ void ens_search_fixed(gs_ensemble_s* e, float* px, float* py, float* pz, const u
     ko.seed_other = seed_other;
     ko.out_map = e->new_to_old.p;
     ko.box = e->box[e->box_cur].p;
-    GS_E_KNN(N, e->k, e->spos.p, e->start.p, e->new_to_old.p, e->old_to_new.p, ko,
-                                      e->walls[9].p, e->walls[10].p, e->walls[11].p, e->obs[0].p, e->obs[1].p,
-                                      e->obs[2].p);
-    GS_LAUNCHED("e_knn");
+    ens_search(e, ko, N <= kTeamMaxCalib ? team_lanes(N, e->k) : 1, st);
 }
 
 // One step, queued on the ensemble's stream (capturable: kernels only).
@@ -687,10 +786,7 @@ void ens_step(gs_ensemble_s* e) {
     ko.seed_other = e->seeded ? e->knn_other[e->kcur].p : nullptr;
     ko.out_map = nullptr;
     ko.box = e->box[e->box_cur].p;
-    GS_E_KNN(N, e->k, e->spos.p, e->start.p, e->new_to_old.p, e->old_to_new.p, ko,
-                                      e->walls[9].p, e->walls[10].p, e->walls[11].p, e->obs[0].p, e->obs[1].p,
-                                      e->obs[2].p);
-    GS_LAUNCHED("e_knn");
+    ens_search(e, ko, step_lanes(e), st);
     e->kcur ^= 1;
     e->seeded = true;
     const Agents A = ens_agents(e);

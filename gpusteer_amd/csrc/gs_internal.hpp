@@ -466,6 +466,10 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
 // reads only the indices before the next search).
 void launch_knn_binned(gs_group_s* A, gs_knn_s* out, gs_group_s* B, uint32_t search_radius, float cap2,
                        const uint32_t* seed, const uint32_t* row_map, const uint32_t* val_map, bool dist = true);
+// The same search by several lanes per query, where A's query count asks for
+// it (returns whether it did).
+bool launch_knn_team(gs_group_s* A, gs_knn_s* out, gs_group_s* B, uint32_t search_radius, float cap2,
+                     const uint32_t* seed, const uint32_t* row_map, const uint32_t* val_map, bool dist);
 void launch_knn_brute(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2);
 // The binned search's semantics (position snapshots of both builds) by an
 // exhaustive scan, for small B.

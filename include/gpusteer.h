@@ -345,7 +345,8 @@ int gs_clear_bits(gs_group A);
  * launch shape the caller may set per context: block_threads in {128, 256,
  * 512} threads per block and agents_per_lane in {1, 2} (a lane handles that
  * many agent slots, so a wavefront covers 64 x agents_per_lane agents).
- * Default 256 x 1.  Results do not depend on the shape.  gpusteer_amd's
+ * Default 256 x 1; smaller groups are searched by several lanes per query
+ * unless another search shape is set.  Results do not depend on the shape.  gpusteer_amd's
  * autotuner picks the shapes by timing them on the workload.  Other values
  * return GS_ERR_UNSUPPORTED.  No counterpart in the reference (fixed
  * block size THREADSPERBLOCK = 256, include/OpenSteer/CUDA/CUDAKernelGlobals.cuh:9). */
