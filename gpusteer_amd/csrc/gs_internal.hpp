@@ -6,6 +6,7 @@
 #include <cfloat>
 #include <cstdint>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <stdexcept>
 #include <string>
@@ -229,6 +230,16 @@ __device__ __forceinline__ void st3(float* x, float* y, float* z, uint32_t i, f3
 // ---------------------------------------------------------------------------
 // Handles.
 namespace gs {
+// Staging of a context's host transfers: a device buffer and a pinned host
+// buffer of up to kStageWords words each, kept between calls and freed with
+// the context.  A transfer holds the mutex until its last copy has ended.
+constexpr size_t kStageWords = (size_t)2 << 20;  // 8 MiB
+struct Staging {
+    std::mutex mu;
+    uint32_t* host = nullptr;
+    uint32_t* dev = nullptr;
+    size_t host_words = 0, dev_words = 0;
+};
 // Launch shape of a tuned kernel: threads per block and agent slots per lane.
 struct LaunchShape {
     uint32_t block = 256;
@@ -241,6 +252,7 @@ struct gs_context_s {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     gs::LaunchShape shape[2];  // GS_SHAPE_KNN, GS_SHAPE_FLOCK
+    gs::Staging stage;
     uint32_t magic = 0x67736378u;
 };
 
@@ -537,6 +549,20 @@ void launch_flock_update(gs_group_s* A, gs_knn_s* knn, const gs_boids_params* p,
 // Whether the fused step may build lazily (steering and bits zero, per-agent
 // constants uniform).
 bool flock_step_lazy_ok(const gs_group_s* A);
+// Fields as words, for the packed host transfers (gs_transfer.hip): the 23
+// float fields and the bits.
+constexpr int kMaxWords = kFields + 1;
+struct FieldWords {
+    uint32_t* p[kMaxWords];
+    int nf;
+};
+// out[f][id of s] = f.p[f][s]; *bad = 1 when an id is out of range.
+void launch_pack_fields(uint32_t n, const uint32_t* ids, const FieldWords& f, uint32_t* out, uint32_t* bad,
+                        hipStream_t st);
+// f.p[f][i] = in[f][i].
+void launch_unpack_fields(uint32_t n, const uint32_t* in, const FieldWords& f, hipStream_t st);
+void launch_pack_knn(uint32_t n, uint32_t nb, uint32_t j0, uint32_t rows, const uint32_t* idx, const float* dist,
+                     const uint32_t* ida, const uint32_t* idb, uint32_t* out, hipStream_t st);
 // Inverts the id map into slot_of_id.
 void launch_invert_ids(gs_group_s* g);
 // Allocation-free KNN (gs_noalloc.hip): locates the fixed scratch array on
