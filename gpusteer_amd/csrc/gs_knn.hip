@@ -1,6 +1,7 @@
-// Exact k-nearest-neighbour search, binned and brute force.
+// Exact k-nearest-neighbour search through the bins (brute force:
+// gs_knn_brute.hip).
 //
-// Semantics (both kernels): for each query a of group A, the k points b of
+// Semantics (both): for each query a of group A, the k points b of
 // group B with the smallest key (d2, b), d2 = ((ax-bx)^2 + (ay-by)^2) + (az-bz)^2
 // in fp32, excluding a itself when A and B are the same group.  This is the
 // order KNNBruteForceCUDAKernelV2 produces (strict '<' over an ascending scan:
@@ -86,47 +87,6 @@ __global__ __launch_bounds__(BS, RF == 1 ? (KMAX <= 8 ? 5 : (KMAX <= 16 ? 4 : 1)
         }
         h.store(k, nA, s, out_idx, out_dist);
     }
-}
-
-// Brute force: one lane per query slot, B staged through LDS in tiles of one
-// block (positions and agent indices).
-template <int KMAX>
-__global__ __launch_bounds__(kBlock) void k_knn_brute(uint32_t nA, const float* __restrict__ ax,
-                                                      const float* __restrict__ ay, const float* __restrict__ az,
-                                                      uint32_t nB, const float* __restrict__ bx,
-                                                      const float* __restrict__ by, const float* __restrict__ bz,
-                                                      const uint32_t* __restrict__ bids, int self, uint32_t k,
-                                                      float cap2, uint32_t* __restrict__ out_idx,
-                                                      float* __restrict__ out_dist) {
-    __shared__ float tx[kBlock], ty[kBlock], tz[kBlock];
-    __shared__ uint32_t tid[kBlock];
-    const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = q < nA;
-    const float qx = active ? ax[q] : 0.f, qy = active ? ay[q] : 0.f, qz = active ? az[q] : 0.f;
-    TopK<KMAX> h;
-    h.init(k);
-    for (uint32_t base = 0; base < nB; base += kBlock) {
-        const uint32_t t = base + threadIdx.x;
-        if (t < nB) {
-            tx[threadIdx.x] = bx[t];
-            ty[threadIdx.x] = by[t];
-            tz[threadIdx.x] = bz[t];
-            tid[threadIdx.x] = bids[t];
-        }
-        __syncthreads();
-        const uint32_t m = min((uint32_t)kBlock, nB - base);
-        if (active) {
-            for (uint32_t j = 0; j < m; ++j) {
-                const uint32_t b = base + j;
-                if (self && b == q) continue;
-                const float d2 = sqdist(qx, qy, qz, tx[j], ty[j], tz[j]);
-                const uint64_t kk = make_key(d2, tid[j]);
-                if (d2 <= cap2 && h.accepts(kk)) h.push(kk, b);
-            }
-        }
-        __syncthreads();
-    }
-    if (active) h.store(k, nA, q, out_idx, out_dist);
 }
 
 // Binned-database semantics over a small or sparse B (walls, obstacles):
@@ -291,22 +251,6 @@ void launch_knn_binned(gs_group_s* A, gs_knn_s* out, gs_group_s* B, uint32_t sea
     else if (out->k <= 8) run_binned_rf<8>(A, out, B, search_radius, cap2, seed, row_map, val_map, dist);
     else if (out->k <= 16) run_binned_rf<16>(A, out, B, search_radius, cap2, seed, row_map, val_map, dist);
     else run_binned_rf<32>(A, out, B, search_radius, cap2, seed, row_map, val_map, dist);
-}
-
-void launch_knn_brute(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2) {
-    const uint32_t nA = A->n;
-    if (nA == 0) return;
-    hipStream_t st = A->ctx->stream;
-    const int self = A == B ? 1 : 0;
-#define GS_BRUTE(KM)                                                                                              \
-    k_knn_brute<KM><<<blocks_for(nA), kBlock, 0, st>>>(nA, A->F(0), A->F(1), A->F(2), B->n, B->F(0), B->F(1),    \
-                                                       B->F(2), B->ids(), self, out->k, cap2, out->idx_alt(),    \
-                                                       out->dist_alt())
-    if (out->k <= 8) GS_BRUTE(8);
-    else if (out->k <= 16) GS_BRUTE(16);
-    else GS_BRUTE(32);
-#undef GS_BRUTE
-    GS_LAUNCHED("k_knn_brute");
 }
 
 void launch_knn_remap(gs_knn_s* out, uint32_t nA, const uint32_t* row_map, const uint32_t* val_map) {
