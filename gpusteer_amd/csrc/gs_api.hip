@@ -1580,7 +1580,7 @@ static bool boids_step_once(gs_group_s* A, gs_knn_s* knn, gs_bins_s* bins, const
     hipStream_t st = A->ctx->stream;
     if (ev) GS_HIP(hipEventRecord(ev[0], st));
     const bool lazy = flock_step_lazy_ok(A);
-    launch_bins_build(A, bins, p->wrap_shape, p->wrap_center, p->wrap_size, lazy, keys_ready);
+    launch_bins_build(A, bins, p->wrap_shape, p->wrap_center, p->wrap_size, lazy, keys_ready, next);
     after_reorder(A);
     if (ev) GS_HIP(hipEventRecord(ev[1], st));
     const Seed sd = seed_for(knn, A, A, p->knn_flags);

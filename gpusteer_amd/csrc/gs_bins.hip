@@ -8,7 +8,9 @@
 // Passes (all over storage slots, coalesced):
 //   1. key      cell per point + atomic arrival rank within the cell (+ optional wrap)
 //   2. scan     exclusive scan of the per-cell counts -> start[C+1]; clears counts
-//   3. scatter  id_tmp[start[cell] + rank] = agent index (the arrival order)
+//   3. scatter  id_tmp[start[cell] + rank] = agent index (the arrival order);
+//               with pass 2 in one block for small groups and lattices, left
+//               out where the order inside a cell is free (k_reorder_free)
 //   4. reorder  per old slot: its final slot puts the members of each cell in
 //               ascending agent index (a stable sort by cell, as thrust's);
 //               every live field, the bits and the agent index are written
@@ -190,6 +192,60 @@ __global__ __launch_bounds__(kBlock) void k_scan_add(uint32_t C, const uint32_t*
     if (fused && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) start[C] = add + partial[blockIdx.x];
 }
 
+// Passes 2 (and 3) of a small lattice in one block: each thread scans a run of
+// consecutive counts, clears them, and with n > 0 the block then scatters the
+// agent indices as k_scatter does.  Bound by latency: 4,096 cells and agents
+// 7.7 us, for launches of 4.7 (tiles), 4.6 (add) and 4.6 us (scatter).
+constexpr int kScanOneThreads = 1024;
+constexpr uint32_t kScanOneCells = 16 * kScanOneThreads;
+constexpr uint32_t kScanOneAgents = 16 * kScanOneThreads;
+__global__ __launch_bounds__(kScanOneThreads) void k_scan_one(uint32_t C, uint32_t* __restrict__ count,
+                                                              uint32_t* start, uint32_t n,
+                                                              const uint32_t* __restrict__ key,
+                                                              const uint32_t* __restrict__ rank,
+                                                              const uint32_t* __restrict__ ids,
+                                                              uint32_t* __restrict__ id_tmp) {
+    __shared__ uint32_t lds[kScanOneThreads / 64];
+    const uint32_t per = (C + kScanOneThreads - 1) / kScanOneThreads;  // at most 16
+    const uint32_t c0 = threadIdx.x * per;
+    uint32_t v[16], sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 16; ++j) {
+        v[j] = (j < per && c0 + j < C) ? count[c0 + j] : 0u;
+        sum += v[j];
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t inc = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t t = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += t;
+    }
+    if (lane == 63) lds[wave] = inc;
+    __syncthreads();
+    uint32_t off = inc - sum, total = 0;
+#pragma unroll
+    for (int w = 0; w < kScanOneThreads / 64; ++w) {
+        off += w < wave ? lds[w] : 0u;
+        total += lds[w];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 16; ++j) {
+        if (j < per && c0 + j < C) {
+            start[c0 + j] = off;
+            count[c0 + j] = 0u;
+        }
+        off += v[j];
+    }
+    if (threadIdx.x == 0) start[C] = total;
+    if (n == 0) return;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += kScanOneThreads) {
+        const uint32_t t = start[key[i]] + rank[i];
+        if (t < n) id_tmp[t] = ids[i];
+    }
+}
+
 // Pass 3: the agent index of every slot of the arrival order (slot t =
 // start[cell] + arrival rank), which the reorder's canonical ranks read.
 __global__ __launch_bounds__(kBlock) void k_scatter(uint32_t n, const uint32_t* __restrict__ key,
@@ -207,7 +263,8 @@ __global__ __launch_bounds__(kBlock) void k_scatter(uint32_t n, const uint32_t* 
 // Pass 4, one lane per old slot s (every read coalesced, the writes land
 // near s since agents rarely change cells): the agent's arrival slot is
 // t = start[cell] + rank, its final slot the cell start plus the number of
-// members of its cell with a smaller agent index.
+// members of its cell with a smaller agent index (id_tmp NULL: the order
+// inside a cell is free, and the arrival slot is final).
 __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint32_t* __restrict__ rank,
                                                     const uint32_t* __restrict__ id_tmp,
                                                     const uint32_t* __restrict__ key,
@@ -226,9 +283,16 @@ __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint32_t* 
     if (t >= n) return;  // only after a corrupted build (see k_scatter)
     const uint32_t id = ids[s];
     uint32_t d = t;
-    if (e - b <= kCanonCap) {
+    if (id_tmp && e - b <= kCanonCap) {
+        // Eight members at a time, so that a crowded cell's reads overlap.
         uint32_t r = 0;
-        for (uint32_t j = b; j < e; ++j) r += (id_tmp[j] < id) ? 1u : 0u;
+        for (uint32_t j = b; j < e; j += 8) {
+            uint32_t o[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) o[u] = id_tmp[min(j + u, e - 1u)];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) r += (j + u < e && o[u] < id) ? 1u : 0u;
+        }
         d = b + r;
     }
     new_to_old[d] = s;
@@ -244,7 +308,89 @@ __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint32_t* 
     if (sfwd) sfwd[d] = make_float4(fs.src[3][s], fs.src[4][s], fs.src[5][s], fs.src[6][s]);
 }
 
+// Passes 2 and 4 of a lazy build whose order inside a cell is free (a step of
+// a call that steps again: results never depend on it, and the call's last
+// step restores the canonical order): an agent's slot is its cell's start plus
+// its arrival rank, so the scatter pass is not needed, and the tile offsets
+// are added here.  Bound by memory (52 bytes read and written per agent) and
+// launches: 1,048,576 agents on 524,288 cells, scan_add + scatter + reorder 5.1
+// + 5.3 + 21.7 us, here 20.0 us.  `off` holds each cell's offset within its scan tile and
+// partial the tile sums; every block scans those itself.  Blocks past the
+// agents' write the cells' starts and clear the counts.
+__global__ __launch_bounds__(kBlock) void k_reorder_free(uint32_t n, uint32_t C, uint32_t ntiles,
+                                                         const uint32_t* __restrict__ rank,
+                                                         const uint32_t* __restrict__ key,
+                                                         const uint32_t* __restrict__ off,
+                                                         const uint32_t* __restrict__ partial,
+                                                         const uint32_t* __restrict__ ids,
+                                                         uint32_t* __restrict__ ids_new,
+                                                         uint32_t* __restrict__ new_to_old,
+                                                         uint32_t* __restrict__ old_to_new, FieldSet fs,
+                                                         float4* __restrict__ spos, float4* __restrict__ sfwd,
+                                                         uint32_t* __restrict__ start, uint32_t* __restrict__ count) {
+    __shared__ uint32_t lds[kBlock / 64];
+    __shared__ uint32_t tile[kScanFusedTiles];
+    const uint32_t agent_blocks = (n + kBlock - 1) / kBlock;
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    // The agent's loads first: they overlap the scan of the tile sums.
+    const bool active = blockIdx.x < agent_blocks && s < n;
+    uint32_t c = 0, t = 0, id = 0;
+    float4 p, f;
+    if (active) {
+        c = key[s];
+        t = off[c] + rank[s];
+        id = ids[s];
+        p = make_float4(fs.src[0][s], fs.src[1][s], fs.src[2][s], __uint_as_float(id));
+        f = make_float4(fs.src[3][s], fs.src[4][s], fs.src[5][s], fs.src[6][s]);
+    }
+    // Exclusive scan of the tile sums, four per thread.
+    constexpr uint32_t kPer = kScanFusedTiles / kBlock;
+    uint32_t v[kPer], sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j) {
+        const uint32_t i = threadIdx.x * kPer + j;
+        v[j] = i < ntiles ? partial[i] : 0u;
+        sum += v[j];
+    }
+    uint32_t total;
+    uint32_t o = block_exclusive_scan(sum, lds, total);
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j) {
+        tile[threadIdx.x * kPer + j] = o;
+        o += v[j];
+    }
+    __syncthreads();
+    if (blockIdx.x < agent_blocks) {
+        if (!active) return;
+        t += tile[c / kScanTile];
+        if (t >= n) return;  // only after a corrupted count array (see k_scatter)
+        new_to_old[t] = s;
+        old_to_new[s] = t;
+        ids_new[t] = id;
+        spos[t] = p;
+        sfwd[t] = f;
+        return;
+    }
+    const uint32_t b = blockIdx.x - agent_blocks;
+    const uint32_t add = tile[b];
+    const uint64_t base = (uint64_t)b * kScanTile;
+#pragma unroll
+    for (int j = 0; j < kScanItems; ++j) {
+        const uint64_t i = base + (uint64_t)j * kBlock + threadIdx.x;
+        if (i < C) {
+            start[i] = off[i] + add;
+            count[i] = 0u;
+        }
+    }
+    if (b == 0 && threadIdx.x == 0) start[C] = total;
+}
+
 void launch_scan_counts(uint32_t* count, uint32_t* start, uint32_t C, hipStream_t st) {
+    if (C <= kScanOneCells) {
+        k_scan_one<<<1, kScanOneThreads, 0, st>>>(C, count, start, 0, nullptr, nullptr, nullptr, nullptr);
+        GS_LAUNCHED("k_scan_one");
+        return;
+    }
     const uint32_t ntiles = (C + kScanTile - 1) / kScanTile;
     uint32_t* partial = start + C + 1;
     k_scan_tiles<<<ntiles, kBlock, 0, st>>>(C, count, start, partial);
@@ -261,10 +407,12 @@ void launch_scan_counts(uint32_t* count, uint32_t* start, uint32_t C, hipStream_
 void launch_scatter_reorder(uint32_t n, const uint32_t* key, const uint32_t* rank, const uint32_t* start,
                             const uint32_t* ids, uint32_t* ids_new, uint32_t* id_tmp,
                             uint32_t* new_to_old, uint32_t* old_to_new, const uint32_t* bits, uint32_t* bits_new,
-                            const FieldSet& fs, float4* spos, hipStream_t st, float4* sfwd) {
+                            const FieldSet& fs, float4* spos, hipStream_t st, float4* sfwd, bool scattered) {
     if (n == 0) return;
-    k_scatter<<<blocks_for(n), kBlock, 0, st>>>(n, key, rank, start, ids, id_tmp);
-    GS_LAUNCHED("k_scatter");
+    if (!scattered) {
+        k_scatter<<<blocks_for(n), kBlock, 0, st>>>(n, key, rank, start, ids, id_tmp);
+        GS_LAUNCHED("k_scatter");
+    }
     k_reorder<<<blocks_for(n), kBlock, 0, st>>>(n, rank, id_tmp, key, start, ids, ids_new, new_to_old,
                                                 old_to_new, bits, bits_new, fs, spos, sfwd);
     GS_LAUNCHED("k_reorder");
@@ -275,7 +423,7 @@ void launch_scatter_reorder(uint32_t n, const uint32_t* key, const uint32_t* ran
 // other field stays in the previous order until the flock kernel, which reads
 // it through new_to_old and writes the step's results in the new order.
 void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const float* wc, const float* ws,
-                       bool lazy, bool keys_ready) {
+                       bool lazy, bool keys_ready, bool free_order) {
     const uint32_t n = g->n;
     const uint32_t C = b->cells;
     hipStream_t st = g->ctx->stream;
@@ -291,6 +439,10 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
     g->spos.reserve(n);
     const uint32_t ntiles = (C + kScanTile - 1) / kScanTile;
     g->start.reserve((size_t)C + 1 + ntiles);  // partial tile sums live after start[C]
+    free_order = free_order && lazy && n > 0;
+    // With k_reorder_free the offsets within the tiles use the scatter's
+    // buffer.
+    const bool free_tiles = free_order && C > kScanOneCells && C <= n && ntiles <= kScanFusedTiles;
     if (new_cells) {
         g->count.reserve(C);
         // A fill kernel rather than hipMemsetAsync, so the build can be
@@ -317,8 +469,29 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
                                                     wsv[2], box_acc, box_clear);
         GS_LAUNCHED("k_bin_key");
     }
-    launch_scan_counts(g->count.p, g->start.p, C, st);
-    if (n > 0) {
+    // Small groups on small lattices: scan and scatter in one launch.
+    const bool one = n > 0 && n <= kScanOneAgents && C <= kScanOneCells && !free_order;
+    if (one) {
+        k_scan_one<<<1, kScanOneThreads, 0, st>>>(C, g->count.p, g->start.p, n, g->key.p, g->rank.p, g->ids(),
+                                                  g->id_tmp.p);
+        GS_LAUNCHED("k_scan_one");
+    } else if (free_tiles) {
+        uint32_t *partial = g->start.p + C + 1, *off = g->id_tmp.p;
+        k_scan_tiles<<<ntiles, kBlock, 0, st>>>(C, g->count.p, off, partial);
+        GS_LAUNCHED("k_scan_tiles");
+        FieldSet fs{};
+        for (int f = 0; f < 7; ++f) fs.src[f] = g->F(f);
+        g->sfwd.reserve(n);
+        k_reorder_free<<<blocks_for(n) + ntiles, kBlock, 0, st>>>(n, C, ntiles, g->rank.p, g->key.p, off, partial,
+                                                                  g->ids(), g->ids_alt(), g->new_to_old.p,
+                                                                  g->old_to_new.p, fs, g->spos.p, g->sfwd.p,
+                                                                  g->start.p, g->count.p);
+        GS_LAUNCHED("k_reorder_free");
+        g->icur ^= 1;
+    } else {
+        launch_scan_counts(g->count.p, g->start.p, C, st);
+    }
+    if (n > 0 && !free_tiles) {
         FieldSet fs{};
         int nf = 0;
         // Fields holding one value in every slot are unchanged by any
@@ -337,10 +510,11 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
             g->sfwd.reserve(n);
         }
         const bool has_bits = !lazy && g->kind == GS_KIND_AGENTS && !g->bits_zero;
-        launch_scatter_reorder(n, g->key.p, g->rank.p, g->start.p, g->ids(), g->ids_alt(), g->id_tmp.p,
+        launch_scatter_reorder(n, g->key.p, g->rank.p, g->start.p, g->ids(), g->ids_alt(),
+                               free_order ? nullptr : g->id_tmp.p,
                                g->new_to_old.p, g->old_to_new.p, has_bits ? g->bits() : nullptr,
                                has_bits ? g->bitsb[g->bcur ^ 1].p : nullptr, fs, g->spos.p, st,
-                               lazy ? g->sfwd.p : nullptr);
+                               lazy ? g->sfwd.p : nullptr, one || free_order);
         for (int f = 0; f < kFields; ++f)
             if (moved & (1u << f)) g->flip(f);
         if (has_bits) g->bcur ^= 1;

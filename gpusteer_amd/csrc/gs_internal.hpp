@@ -456,11 +456,12 @@ __device__ __forceinline__ void count_and_rank(bool active, uint32_t c, uint32_t
 void launch_scan_counts(uint32_t* count, uint32_t* start, uint32_t C, hipStream_t st);
 // Stable scatter of n keyed slots into cell order and the gather of every
 // field in fs, bits and ids into the new order; writes the order maps and
-// the packed position snapshot.
+// the packed position snapshot.  scattered: id_tmp is already filled.
 void launch_scatter_reorder(uint32_t n, const uint32_t* key, const uint32_t* rank, const uint32_t* start,
                             const uint32_t* ids, uint32_t* ids_new, uint32_t* id_tmp,
                             uint32_t* new_to_old, uint32_t* old_to_new, const uint32_t* bits, uint32_t* bits_new,
-                            const FieldSet& fs, float4* spos, hipStream_t st, float4* sfwd = nullptr);
+                            const FieldSet& fs, float4* spos, hipStream_t st, float4* sfwd = nullptr,
+                            bool scattered = false);
 
 // Host-side launchers (one per operation) implemented in the .hip files.
 void launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t st);
@@ -469,8 +470,10 @@ void launch_iota(uint32_t* p, uint32_t n, hipStream_t st);
 // first); also writes the position snapshot spos.
 // keys_ready: the previous step's flock kernel already did the key pass
 // (launch_flock_update's next_bins) for this lattice and wrap.
+// free_order: the order of the agents inside a cell is free (a lazy build
+// that another build of the same call follows).
 void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const float* wc, const float* ws,
-                       bool lazy = false, bool keys_ready = false);
+                       bool lazy = false, bool keys_ready = false, bool free_order = false);
 // KNN into out's alternate buffer (caller flips).  row_map / val_map translate
 // a seed held at the previous storage order of A / B (NULL: same order).
 // cap2: only points with d2 <= cap2 qualify (+inf: no cap).
