@@ -36,6 +36,7 @@ void hip_check(hipError_t e, const char* what) {
 // Frame recording on this thread (gs_frame_begin .. gs_frame_end), or NULL.
 struct Recording;
 static thread_local Recording* t_rec = nullptr;
+bool recording_frame() { return t_rec != nullptr; }
 // Fails a call that cannot be recorded into a frame while one is recorded.
 static void no_frame(const char* what) {
     if (t_rec)
@@ -432,6 +433,10 @@ static void visit(gs_group_s* g, SnapIO& io) {
     io.val(g->bbox_wanted);
     io.val(g->bbox_fresh);
     for (auto& b : g->bbox) io.buf(b);
+    io.buf(g->cbox);
+    // Not compared: a recorded search computes the chunk boxes it reads, and
+    // after a recording or a replay they are computed anew.
+    if (io.write) g->cbox_fresh = false;
 }
 
 static void visit(gs_knn_s* k, SnapIO& io) {
@@ -742,6 +747,7 @@ static void release_group(gs_group_s* g) {
     g->spos.release();
     g->sfwd.release();
     for (auto& b : g->bbox) b.release();
+    g->cbox.release();
 }
 
 int gs_group_destroy(gs_group g) {
@@ -779,6 +785,9 @@ static void begin_members(gs_group_s* g, uint32_t n) {
     g->idb[0].reserve(n);
     g->idb[1].reserve(n);
     g->slot_of_id.reserve(n);
+    // Here rather than at the first search, which may be recorded into a frame.
+    if (n <= kChunkMax) g->cbox.reserve(chunk_words(kChunkMax));
+    g->cbox_fresh = false;
     launch_iota(g->ids(), n, g->ctx->stream);
     g->n = n;
     g->inv = 0;
@@ -1268,10 +1277,16 @@ static void find_knn(gs_group A, gs_knn out, gs_bins bins, gs_group B, uint32_t 
     // B's builds from now on keep its bounding box, which lets the binned
     // search skip queries the cap cannot reach it from.
     if (std::isfinite(cap2)) B->bbox_wanted = true;
-    if (!(flags & GS_KNN_BINNED) && prefer_split(A, B, bins->g, bins->cells, max_distance)) {
+    const bool split = !(flags & GS_KNN_BINNED) && prefer_split(A, B, bins->g, bins->cells, max_distance);
+    const bool exhaustive =
+        !split && !(flags & GS_KNN_BINNED) && prefer_exhaustive(B, bins->g, bins->cells, max_distance);
+    if ((split || exhaustive) && out->k <= kChunkMaxK && B->n <= kChunkMax) {
+        const Seed sd = seed_for(out, A, B, flags);
+        launch_knn_chunks(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map);
+    } else if (split) {
         const Seed sd = seed_for(out, A, B, flags);
         launch_knn_split(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map);
-    } else if (!(flags & GS_KNN_BINNED) && prefer_exhaustive(B, bins->g, bins->cells, max_distance)) {
+    } else if (exhaustive) {
         launch_knn_snap_brute(A, out, B, cap2);
     } else {
         const Seed sd = seed_for(out, A, B, flags);

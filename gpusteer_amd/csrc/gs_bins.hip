@@ -463,6 +463,7 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
         box_clear = g->bbox[g->bbox_cur ^ 1].p;
     }
     g->bbox_fresh = box_acc != nullptr;
+    g->cbox_fresh = false;
     if (n > 0 && !keys_ready) {
         k_bin_key<<<blocks_for(n), kBlock, 0, st>>>(n, g->F(0), g->F(1), g->F(2), b->g, g->key.p, g->rank.p,
                                                     g->count.p, wrap_shape, wcv[0], wcv[1], wcv[2], wsv[0], wsv[1],

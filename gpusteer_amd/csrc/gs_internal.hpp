@@ -336,6 +336,11 @@ struct gs_group_s {
     uint8_t bbox_cur = 0;
     bool bbox_wanted = false;
     bool bbox_fresh = false;
+    // Bounding boxes of the snapshot's 64-slot chunks, for the exhaustive
+    // searches of small groups (launch_knn_chunks; groups of at most
+    // kChunkMax points).  cbox_fresh: they are the current snapshot's.
+    gs::DevBuf<float> cbox;
+    bool cbox_fresh = false;
 
     float* F(int j) const { return fb[j][fcur[j]].p; }
     float* Falt(int j) const { return fb[j][fcur[j] ^ 1].p; }
@@ -510,6 +515,20 @@ constexpr uint32_t kSplitWaves = 4096;
 constexpr uint32_t kSplitMinRange = 64;
 constexpr uint64_t kSplitMinCells = 64;
 constexpr int kSplitBuf = 16;  // deferred entries per lane
+// The exhaustive scans of B by teams of lanes over B's 64-slot chunks, skipping
+// chunks beyond the query's bound; lists of up to kChunkMaxK.
+constexpr uint32_t kChunkMax = 16384;
+constexpr uint32_t kChunkMaxK = 16;
+// Words of cbox for n points: min x, y, z, max x, y, z and the points that are
+// numbers, per chunk.
+constexpr size_t chunk_words(uint32_t n) { return 7 * (((size_t)n + 63) / 64); }
+void launch_knn_chunks(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, const uint32_t* seed,
+                       const uint32_t* row_map, const uint32_t* val_map);
+// The chunk boxes of B's snapshot, if they are not the current one's.
+void launch_chunk_boxes(gs_group_s* B);
+// Whether this thread records a frame (its kernels run at the replays, so
+// nothing that a call finds done may be left out of it).
+bool recording_frame();
 // Number of ranges for nA queries over nB points (< 2: no split).
 uint32_t knn_split_ranges(uint32_t nA, uint32_t nB);
 // The split exhaustive scan (falls back to the unsplit one below 2 ranges);

@@ -31,13 +31,7 @@ __global__ __launch_bounds__(kBlock) void k_knn_team(uint32_t nA, const float4* 
         const FlatQuery Q{q.x, q.y, q.z, thr, self ? s : UINT32_MAX, active};
         knn_search_team(L, Q, g, nB, bpos, bstart);
     }
-    if (!active) return;
-    for (uint32_t j = L.lane; j < k; j += G) {
-        const size_t o = (size_t)j * nA + s;
-        const bool pad = (int)j >= L.cnt;
-        out_idx[o] = pad ? UINT32_MAX : L.best_slot[j];
-        if (out_dist) out_dist[o] = pad ? FLT_MAX : sqrtf(__uint_as_float((uint32_t)(L.best_key[j] >> 32)));
-    }
+    if (active) L.store(nA, s, out_idx, out_dist);
 }
 
 // Bound by the serial chain of one team (seven dependent loads: query, seed,

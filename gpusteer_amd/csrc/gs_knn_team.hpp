@@ -210,6 +210,18 @@ template <int G, int KM, int RF> struct TeamList {
         cnt += __popc(v);
     }
 
+    // The sorted list to column `row` of the slot-major [k][n] output (pads
+    // UINT32_MAX / FLT_MAX); no distances when out_dist is NULL.
+    __device__ __forceinline__ void store(uint32_t n, uint32_t row, uint32_t* __restrict__ out_idx,
+                                          float* __restrict__ out_dist) const {
+        for (uint32_t j = lane; j < k; j += G) {
+            const size_t o = (size_t)j * n + row;
+            const bool pad = (int)j >= cnt;
+            out_idx[o] = pad ? UINT32_MAX : best_slot[j];
+            if (out_dist) out_dist[o] = pad ? FLT_MAX : sqrtf(__uint_as_float((uint32_t)(best_key[j] >> 32)));
+        }
+    }
+
     // A bound on the k-th distance from the M runs: each lane's two nearest
     // candidates are 2 G distinct points, and the k-th nearest of them lies
     // no nearer than the k-th of all (+inf with fewer than k).
