@@ -1609,6 +1609,48 @@ static bool boids_step_once(gs_group_s* A, gs_knn_s* knn, gs_bins_s* bins, const
     return fuse;
 }
 
+// Whether a crowd frame can go phase by phase for both groups at once: every
+// call of the sequence below would succeed, the groups are small (so each
+// phase is bound by its launch and its latency), and every list is short and
+// its own container.
+static bool pair_frame_ok(gs_group_s* const A[2], const gs_group_s* W, const gs_group_s* O, const gs_bins_s* bins,
+                          gs_knn_s* const* knn, const gs_scenario* s, float cap) {
+    if (A[0] == A[1] || std::isnan(cap)) return false;
+    const gs_context_s* ctx = A[0]->ctx;
+    if (A[1]->ctx != ctx || W->ctx != ctx || O->ctx != ctx || bins->ctx != ctx) return false;
+    for (int g = 0; g < 2; ++g)
+        if (!pair_build_ok(A[g], bins)) return false;
+    for (const gs_group_s* b : {W, O})
+        if (!b->binned || !b->snap_valid || !same_grid(b->bin_grid, bins->g) || b->n > kSmallTargetSet) return false;
+    for (int j = 0; j < 8; ++j) {
+        if (knn[j]->ctx != ctx || knn[j]->n != A[j / 4]->n || knn[j]->k > 8) return false;
+        for (int i = 0; i < j; ++i)
+            if (knn[i] == knn[j]) return false;
+    }
+    return true;
+}
+static void pair_frame(gs_group_s* const A[2], gs_group_s* W, gs_group_s* O, gs_bins_s* bins, gs_knn_s* const* knn,
+                       const gs_scenario* s, float cap2) {
+    use_device(A[0]->ctx);
+    for (int g = 0; g < 2; ++g)
+        if (std::isfinite(cap2)) A[g]->bbox_wanted = true;
+    launch_pair_build(A, bins);
+    for (int g = 0; g < 2; ++g) after_reorder(A[g]);
+    ListSeed seeds[4];
+    for (int g = 0; g < 2; ++g)
+        for (int o = 0; o < 2; ++o) {
+            const Seed sd = seed_for(knn[4 * g + o], A[g], A[o ? 1 - g : g], GS_KNN_DEFAULT);
+            seeds[2 * g + o] = ListSeed{sd.seed, sd.row_map, sd.val_map};
+        }
+    launch_pair_search(A, W, O, knn, seeds, cap2);
+    for (int j = 0; j < 8; ++j) {
+        gs_group_s* const b[4] = {A[j / 4], A[1 - j / 4], W, O};
+        knn[j]->cur ^= 1;
+        mark_result(knn[j], A[j / 4], b[j % 4]);
+    }
+    launch_pair_steer(A, W, O, knn, s);
+}
+
 int gs_step_choke(gs_group A0, gs_group A1, gs_group walls, gs_group obstacles, gs_bins bins, gs_knn const* knn,
                   const gs_scenario* s, uint32_t steps) {
     return guarded([&] {
@@ -1629,6 +1671,10 @@ int gs_step_choke(gs_group A0, gs_group A1, gs_group walls, gs_group obstacles, 
         const gs_flock_term& t = s->choke_separation;
         const float cap = s->other_max_distance > 0.f ? s->other_max_distance : INFINITY;
         for (uint32_t step = 0; step < steps; ++step) {
+            if (pair_frame_ok(A, walls, obstacles, bins, knn, s, cap)) {
+                pair_frame(A, walls, obstacles, bins, knn, s, cap2_of(cap));
+                continue;
+            }
             ok(gs_update_knn_database(A[0], bins));
             ok(gs_update_knn_database(A[1], bins));
             for (int g = 0; g < 2; ++g) {

@@ -18,6 +18,8 @@
 // Because the previous build left the state in cell order and agents move
 // little between builds, the reorder's writes land nearly sequentially.  The counts array is all-zero between builds (pass 2 clears it),
 // so no memset is recorded in the stream.
+#include <algorithm>
+
 #include "gs_internal.hpp"
 
 namespace gs {
@@ -66,12 +68,11 @@ void launch_iota(uint32_t* p, uint32_t n, hipStream_t st) {
     GS_LAUNCHED("k_iota");
 }
 
-__global__ __launch_bounds__(kBlock) void k_bin_key(uint32_t n, float* __restrict__ px, float* __restrict__ py,
-                                                    float* __restrict__ pz, GridDev g, uint32_t* __restrict__ key,
-                                                    uint32_t* __restrict__ rank, uint32_t* __restrict__ count,
-                                                    int wrap_shape, float wcx, float wcy, float wcz, float wsx,
-                                                    float wsy, float wsz, uint32_t* __restrict__ box_acc,
-                                                    uint32_t* __restrict__ box_clear) {
+__device__ __forceinline__ void bin_key(uint32_t n, float* __restrict__ px, float* __restrict__ py,
+                                        float* __restrict__ pz, const GridDev& g, uint32_t* __restrict__ key,
+                                        uint32_t* __restrict__ rank, uint32_t* __restrict__ count, int wrap_shape,
+                                        float wcx, float wcy, float wcz, float wsx, float wsy, float wsz,
+                                        uint32_t* __restrict__ box_acc, uint32_t* __restrict__ box_clear) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = i < n;
     const int lane = threadIdx.x & 63;
@@ -97,6 +98,13 @@ __global__ __launch_bounds__(kBlock) void k_bin_key(uint32_t n, float* __restric
         if (blockIdx.x == 0 && threadIdx.x < 6) box_clear[threadIdx.x] = threadIdx.x < 3 ? kBoxEmptyMin : kBoxEmptyMax;
         box_accumulate(active, x, y, z, box_acc);
     }
+}
+
+__global__ __launch_bounds__(kBlock) void k_bin_key(uint32_t n, float* px, float* py, float* pz, GridDev g,
+                                                    uint32_t* key, uint32_t* rank, uint32_t* count, int wrap_shape,
+                                                    float wcx, float wcy, float wcz, float wsx, float wsy, float wsz,
+                                                    uint32_t* box_acc, uint32_t* box_clear) {
+    bin_key(n, px, py, pz, g, key, rank, count, wrap_shape, wcx, wcy, wcz, wsx, wsy, wsz, box_acc, box_clear);
 }
 
 // Wavefront-then-block exclusive scan of one value per thread.
@@ -199,12 +207,9 @@ __global__ __launch_bounds__(kBlock) void k_scan_add(uint32_t C, const uint32_t*
 constexpr int kScanOneThreads = 1024;
 constexpr uint32_t kScanOneCells = 16 * kScanOneThreads;
 constexpr uint32_t kScanOneAgents = 16 * kScanOneThreads;
-__global__ __launch_bounds__(kScanOneThreads) void k_scan_one(uint32_t C, uint32_t* __restrict__ count,
-                                                              uint32_t* start, uint32_t n,
-                                                              const uint32_t* __restrict__ key,
-                                                              const uint32_t* __restrict__ rank,
-                                                              const uint32_t* __restrict__ ids,
-                                                              uint32_t* __restrict__ id_tmp) {
+__device__ __forceinline__ void scan_one(uint32_t C, uint32_t* __restrict__ count, uint32_t* start, uint32_t n,
+                                         const uint32_t* __restrict__ key, const uint32_t* __restrict__ rank,
+                                         const uint32_t* __restrict__ ids, uint32_t* __restrict__ id_tmp) {
     __shared__ uint32_t lds[kScanOneThreads / 64];
     const uint32_t per = (C + kScanOneThreads - 1) / kScanOneThreads;  // at most 16
     const uint32_t c0 = threadIdx.x * per;
@@ -246,6 +251,12 @@ __global__ __launch_bounds__(kScanOneThreads) void k_scan_one(uint32_t C, uint32
     }
 }
 
+__global__ __launch_bounds__(kScanOneThreads) void k_scan_one(uint32_t C, uint32_t* count, uint32_t* start, uint32_t n,
+                                                              const uint32_t* key, const uint32_t* rank,
+                                                              const uint32_t* ids, uint32_t* id_tmp) {
+    scan_one(C, count, start, n, key, rank, ids, id_tmp);
+}
+
 // Pass 3: the agent index of every slot of the arrival order (slot t =
 // start[cell] + arrival rank), which the reorder's canonical ranks read.
 __global__ __launch_bounds__(kBlock) void k_scatter(uint32_t n, const uint32_t* __restrict__ key,
@@ -265,16 +276,13 @@ __global__ __launch_bounds__(kBlock) void k_scatter(uint32_t n, const uint32_t* 
 // t = start[cell] + rank, its final slot the cell start plus the number of
 // members of its cell with a smaller agent index (id_tmp NULL: the order
 // inside a cell is free, and the arrival slot is final).
-__global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint32_t* __restrict__ rank,
-                                                    const uint32_t* __restrict__ id_tmp,
-                                                    const uint32_t* __restrict__ key,
-                                                    const uint32_t* __restrict__ start,
-                                                    const uint32_t* __restrict__ ids, uint32_t* __restrict__ ids_new,
-                                                    uint32_t* __restrict__ new_to_old,
-                                                    uint32_t* __restrict__ old_to_new,
-                                                    const uint32_t* __restrict__ bits, uint32_t* __restrict__ bits_new,
-                                                    FieldSet fs, float4* __restrict__ spos,
-                                                    float4* __restrict__ sfwd) {
+__device__ __forceinline__ void reorder(uint32_t n, const uint32_t* __restrict__ rank,
+                                        const uint32_t* __restrict__ id_tmp, const uint32_t* __restrict__ key,
+                                        const uint32_t* __restrict__ start, const uint32_t* __restrict__ ids,
+                                        uint32_t* __restrict__ ids_new, uint32_t* __restrict__ new_to_old,
+                                        uint32_t* __restrict__ old_to_new, const uint32_t* __restrict__ bits,
+                                        uint32_t* __restrict__ bits_new, const FieldSet& fs,
+                                        float4* __restrict__ spos, float4* __restrict__ sfwd) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
     const uint32_t c = key[s];
@@ -306,6 +314,40 @@ __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint32_t* 
     // snapshots forward and speed (fields 3..6, passed after them)
     spos[d] = make_float4(fs.src[0][s], fs.src[1][s], fs.src[2][s], __uint_as_float(id));
     if (sfwd) sfwd[d] = make_float4(fs.src[3][s], fs.src[4][s], fs.src[5][s], fs.src[6][s]);
+}
+
+__global__ __launch_bounds__(kBlock) void k_reorder(uint32_t n, const uint32_t* rank, const uint32_t* id_tmp,
+                                                    const uint32_t* key, const uint32_t* start, const uint32_t* ids,
+                                                    uint32_t* ids_new, uint32_t* new_to_old, uint32_t* old_to_new,
+                                                    const uint32_t* bits, uint32_t* bits_new, FieldSet fs,
+                                                    float4* spos, float4* sfwd) {
+    reorder(n, rank, id_tmp, key, start, ids, ids_new, new_to_old, old_to_new, bits, bits_new, fs, spos, sfwd);
+}
+
+// The three passes of two small groups' builds on one lattice at once: group
+// blockIdx.y.
+struct PairBuild {
+    struct One {
+        uint32_t n;
+        float *px, *py, *pz;
+        uint32_t *key, *rank, *count, *start, *id_tmp, *ids, *ids_new, *new_to_old, *old_to_new, *box_acc, *box_clear;
+        uint32_t *bits, *bits_new;
+        FieldSet fs;
+        float4* spos;
+    } g[2];
+};
+__global__ __launch_bounds__(kBlock) void k_pair_key(PairBuild P, GridDev g) {
+    const PairBuild::One& b = P.g[blockIdx.y];
+    bin_key(b.n, b.px, b.py, b.pz, g, b.key, b.rank, b.count, -1, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, b.box_acc, b.box_clear);
+}
+__global__ __launch_bounds__(kScanOneThreads) void k_pair_scan(PairBuild P, uint32_t C) {
+    const PairBuild::One& b = P.g[blockIdx.y];
+    scan_one(C, b.count, b.start, b.n, b.key, b.rank, b.ids, b.id_tmp);
+}
+__global__ __launch_bounds__(kBlock) void k_pair_reorder(PairBuild P) {
+    const PairBuild::One& b = P.g[blockIdx.y];
+    reorder(b.n, b.rank, b.id_tmp, b.key, b.start, b.ids, b.ids_new, b.new_to_old, b.old_to_new, b.bits, b.bits_new,
+            b.fs, b.spos, nullptr);
 }
 
 // Passes 2 and 4 of a lazy build whose order inside a cell is free (a step of
@@ -418,6 +460,105 @@ void launch_scatter_reorder(uint32_t n, const uint32_t* key, const uint32_t* ran
     GS_LAUNCHED("k_reorder");
 }
 
+// Buffers of a build of g on b (counts zero for a new lattice), and where its
+// key pass keeps the positions' bounding box once a capped search targets the
+// group (acc NULL: nowhere).
+struct BoxPair {
+    uint32_t *acc, *clear;
+};
+static BoxPair begin_build(gs_group_s* g, const gs_bins_s* b) {
+    const uint32_t n = g->n, C = b->cells;
+    g->key.reserve(n);
+    g->rank.reserve(n);
+    g->id_tmp.reserve(n);
+    g->new_to_old.reserve(n);
+    g->old_to_new.reserve(n);
+    g->spos.reserve(n);
+    g->start.reserve((size_t)C + 1 + (C + kScanTile - 1) / kScanTile);  // partial tile sums live after start[C]
+    if (!g->binned || g->bin_cells != C || g->count.cap < C) {
+        g->count.reserve(C);
+        // A fill kernel rather than hipMemsetAsync, so the build can be
+        // captured into a graph.
+        launch_fill_u32(g->count.p, C, 0u, g->ctx->stream);
+    }
+    g->bin_cells = C;
+    g->bin_grid = b->g;
+    BoxPair box{nullptr, nullptr};
+    if (g->bbox_wanted && g->bbox[0].p && g->bbox[1].p && n > 0) {
+        g->bbox_cur ^= 1;
+        box.acc = g->bbox[g->bbox_cur].p;
+        box.clear = g->bbox[g->bbox_cur ^ 1].p;
+    }
+    g->bbox_fresh = box.acc != nullptr;
+    g->cbox_fresh = false;
+    return box;
+}
+// The fields a build moves.  Fields holding one value in every slot are
+// unchanged by any permutation and stay where they are (positions always
+// move: the snapshot is built from them).
+static uint32_t moved_fields(const gs_group_s* g, FieldSet& fs) {
+    const uint32_t moved = g->live & ~(g->inv & ~kFPos);
+    fs.nf = 0;
+    for (int f = 0; f < kFields; ++f)
+        if (moved & (1u << f)) {
+            fs.src[fs.nf] = g->F(f);
+            fs.dst[fs.nf] = g->Falt(f);
+            ++fs.nf;
+        }
+    return moved;
+}
+static bool moves_bits(const gs_group_s* g) { return g->kind == GS_KIND_AGENTS && !g->bits_zero; }
+static void end_build(gs_group_s* g, uint32_t moved, bool bits) {
+    for (int f = 0; f < kFields; ++f)
+        if (moved & (1u << f)) g->flip(f);
+    if (bits) g->bcur ^= 1;
+    if (g->n > 0) g->icur ^= 1;
+    g->binned = true;
+    g->snap_valid = true;
+}
+
+bool pair_build_ok(const gs_group_s* g, const gs_bins_s* b) {
+    return g->n > 0 && g->n <= kScanOneAgents && b->cells <= kScanOneCells;
+}
+void launch_pair_build(gs_group_s* const g[2], const gs_bins_s* b) {
+    PairBuild P{};
+    uint32_t moved[2], n = 0;
+    bool bits[2];
+    for (int i = 0; i < 2; ++i) {
+        const BoxPair box = begin_build(g[i], b);
+        PairBuild::One& o = P.g[i];
+        o.n = g[i]->n;
+        n = std::max(n, o.n);
+        o.px = g[i]->F(0);
+        o.py = g[i]->F(1);
+        o.pz = g[i]->F(2);
+        o.key = g[i]->key.p;
+        o.rank = g[i]->rank.p;
+        o.count = g[i]->count.p;
+        o.start = g[i]->start.p;
+        o.id_tmp = g[i]->id_tmp.p;
+        o.ids = g[i]->ids();
+        o.ids_new = g[i]->ids_alt();
+        o.new_to_old = g[i]->new_to_old.p;
+        o.old_to_new = g[i]->old_to_new.p;
+        o.box_acc = box.acc;
+        o.box_clear = box.clear;
+        moved[i] = moved_fields(g[i], o.fs);
+        bits[i] = moves_bits(g[i]);
+        o.bits = bits[i] ? g[i]->bits() : nullptr;
+        o.bits_new = bits[i] ? g[i]->bitsb[g[i]->bcur ^ 1].p : nullptr;
+        o.spos = g[i]->spos.p;
+    }
+    hipStream_t st = g[0]->ctx->stream;
+    k_pair_key<<<dim3(blocks_for(n), 2), kBlock, 0, st>>>(P, b->g);
+    GS_LAUNCHED("k_pair_key");
+    k_pair_scan<<<dim3(1, 2), kScanOneThreads, 0, st>>>(P, b->cells);
+    GS_LAUNCHED("k_pair_scan");
+    k_pair_reorder<<<dim3(blocks_for(n), 2), kBlock, 0, st>>>(P);
+    GS_LAUNCHED("k_pair_reorder");
+    for (int i = 0; i < 2; ++i) end_build(g[i], moved[i], bits[i]);
+}
+
 // lazy (fused Boids step only): move nothing but the snapshots (positions,
 // and forward + speed into sfwd), the agent indices and the maps; every
 // other field stays in the previous order until the flock kernel, which reads
@@ -427,47 +568,23 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
     const uint32_t n = g->n;
     const uint32_t C = b->cells;
     hipStream_t st = g->ctx->stream;
-    const bool new_cells = !g->binned || g->bin_cells != C || g->count.cap < C;
     // Keys from the previous step's flock kernel (counts already taken):
     // only for the lattice that step was built on, never with a box to keep.
-    if (keys_ready && (new_cells || g->bbox_wanted)) fail(GS_ERR_INVALID_ARGUMENT, "internal: stale fused keys");
-    g->key.reserve(n);
-    g->rank.reserve(n);
-    g->id_tmp.reserve(n);
-    g->new_to_old.reserve(n);
-    g->old_to_new.reserve(n);
-    g->spos.reserve(n);
+    if (keys_ready && (!g->binned || g->bin_cells != C || g->count.cap < C || g->bbox_wanted))
+        fail(GS_ERR_INVALID_ARGUMENT, "internal: stale fused keys");
+    const BoxPair box = begin_build(g, b);
     const uint32_t ntiles = (C + kScanTile - 1) / kScanTile;
-    g->start.reserve((size_t)C + 1 + ntiles);  // partial tile sums live after start[C]
     free_order = free_order && lazy && n > 0;
     // With k_reorder_free the offsets within the tiles use the scatter's
     // buffer.
     const bool free_tiles = free_order && C > kScanOneCells && C <= n && ntiles <= kScanFusedTiles;
-    if (new_cells) {
-        g->count.reserve(C);
-        // A fill kernel rather than hipMemsetAsync, so the build can be
-        // captured into a graph.
-        launch_fill_u32(g->count.p, C, 0u, st);
-    }
-    g->bin_cells = C;
-    g->bin_grid = b->g;
     float wcv[3] = {0, 0, 0}, wsv[3] = {0, 0, 0};
     if (wc) memcpy(wcv, wc, sizeof wcv);
     if (ws) memcpy(wsv, ws, sizeof wsv);
-    // Bounding box of this build's positions, once a capped search targets
-    // the group.
-    uint32_t *box_acc = nullptr, *box_clear = nullptr;
-    if (g->bbox_wanted && g->bbox[0].p && g->bbox[1].p && n > 0) {
-        g->bbox_cur ^= 1;
-        box_acc = g->bbox[g->bbox_cur].p;
-        box_clear = g->bbox[g->bbox_cur ^ 1].p;
-    }
-    g->bbox_fresh = box_acc != nullptr;
-    g->cbox_fresh = false;
     if (n > 0 && !keys_ready) {
         k_bin_key<<<blocks_for(n), kBlock, 0, st>>>(n, g->F(0), g->F(1), g->F(2), b->g, g->key.p, g->rank.p,
                                                     g->count.p, wrap_shape, wcv[0], wcv[1], wcv[2], wsv[0], wsv[1],
-                                                    wsv[2], box_acc, box_clear);
+                                                    wsv[2], box.acc, box.clear);
         GS_LAUNCHED("k_bin_key");
     }
     // Small groups on small lattices: scan and scatter in one launch.
@@ -488,41 +605,26 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
                                                                   g->old_to_new.p, fs, g->spos.p, g->sfwd.p,
                                                                   g->start.p, g->count.p);
         GS_LAUNCHED("k_reorder_free");
-        g->icur ^= 1;
     } else {
         launch_scan_counts(g->count.p, g->start.p, C, st);
     }
+    uint32_t moved = 0;
+    bool has_bits = false;
     if (n > 0 && !free_tiles) {
         FieldSet fs{};
-        int nf = 0;
-        // Fields holding one value in every slot are unchanged by any
-        // permutation and stay where they are (positions always move: the
-        // snapshot is built from them).
-        const uint32_t moved = lazy ? 0u : g->live & ~(g->inv & ~kFPos);
-        for (int f = 0; f < kFields; ++f)
-            if (moved & (1u << f)) {
-                fs.src[nf] = g->F(f);
-                fs.dst[nf] = g->Falt(f);
-                ++nf;
-            }
-        fs.nf = nf;
         if (lazy) {
             for (int f = 0; f < 7; ++f) fs.src[f] = g->F(f);
             g->sfwd.reserve(n);
+        } else {
+            moved = moved_fields(g, fs);
+            has_bits = moves_bits(g);
         }
-        const bool has_bits = !lazy && g->kind == GS_KIND_AGENTS && !g->bits_zero;
         launch_scatter_reorder(n, g->key.p, g->rank.p, g->start.p, g->ids(), g->ids_alt(),
-                               free_order ? nullptr : g->id_tmp.p,
-                               g->new_to_old.p, g->old_to_new.p, has_bits ? g->bits() : nullptr,
-                               has_bits ? g->bitsb[g->bcur ^ 1].p : nullptr, fs, g->spos.p, st,
-                               lazy ? g->sfwd.p : nullptr, one || free_order);
-        for (int f = 0; f < kFields; ++f)
-            if (moved & (1u << f)) g->flip(f);
-        if (has_bits) g->bcur ^= 1;
-        g->icur ^= 1;
+                               free_order ? nullptr : g->id_tmp.p, g->new_to_old.p, g->old_to_new.p,
+                               has_bits ? g->bits() : nullptr, has_bits ? g->bitsb[g->bcur ^ 1].p : nullptr, fs,
+                               g->spos.p, st, lazy ? g->sfwd.p : nullptr, one || free_order);
     }
-    g->binned = true;
-    g->snap_valid = true;
+    end_build(g, moved, has_bits);
 }
 
 }  // namespace gs

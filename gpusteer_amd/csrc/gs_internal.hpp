@@ -529,6 +529,19 @@ void launch_chunk_boxes(gs_group_s* B);
 // Whether this thread records a frame (its kernels run at the replays, so
 // nothing that a call finds done may be left out of it).
 bool recording_frame();
+// Crowd frames (gs_step_choke) of two small groups, each phase one launch for
+// both: the builds, the eight searches (knn: own group, other group, walls,
+// obstacles of group 0, then of group 1; seeds likewise for the first two of
+// each), the steering and the integrate.
+struct ListSeed {
+    const uint32_t *seed, *row_map, *val_map;
+};
+bool pair_build_ok(const gs_group_s* g, const gs_bins_s* b);
+void launch_pair_build(gs_group_s* const g[2], const gs_bins_s* b);
+void launch_pair_search(gs_group_s* const g[2], gs_group_s* W, gs_group_s* O, gs_knn_s* const knn[8],
+                        const ListSeed seeds[4], float cap2);
+void launch_pair_steer(gs_group_s* const g[2], gs_group_s* W, gs_group_s* O, gs_knn_s* const knn[8],
+                       const gs_scenario* s);
 // Number of ranges for nA queries over nB points (< 2: no split).
 uint32_t knn_split_ranges(uint32_t nA, uint32_t nB);
 // The split exhaustive scan (falls back to the unsplit one below 2 ranges);
