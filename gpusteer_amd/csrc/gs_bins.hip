@@ -203,7 +203,9 @@ __global__ __launch_bounds__(kBlock) void k_scan_add(uint32_t C, const uint32_t*
 // Passes 2 (and 3) of a small lattice in one block: each thread scans a run of
 // consecutive counts, clears them, and with n > 0 the block then scatters the
 // agent indices as k_scatter does.  Bound by latency: 4,096 cells and agents
-// 7.7 us, for launches of 4.7 (tiles), 4.6 (add) and 4.6 us (scatter).
+// 7.7 us, for launches of 4.7 (tiles), 4.6 (add) and 4.6 us (scatter); with
+// counts read and starts written 16 bytes at a time 5.6 us, and 12,167 cells
+// with 5,000 agents 13.5 -> 8.7 us.
 constexpr int kScanOneThreads = 1024;
 constexpr uint32_t kScanOneCells = 16 * kScanOneThreads;
 constexpr uint32_t kScanOneAgents = 16 * kScanOneThreads;
@@ -211,13 +213,24 @@ __device__ __forceinline__ void scan_one(uint32_t C, uint32_t* __restrict__ coun
                                          const uint32_t* __restrict__ key, const uint32_t* __restrict__ rank,
                                          const uint32_t* __restrict__ ids, uint32_t* __restrict__ id_tmp) {
     __shared__ uint32_t lds[kScanOneThreads / 64];
-    const uint32_t per = (C + kScanOneThreads - 1) / kScanOneThreads;  // at most 16
+    // Consecutive counts per thread, a multiple of four (16-byte accesses), at
+    // most 16.
+    const uint32_t per = ((C + kScanOneThreads - 1) / kScanOneThreads + 3u) & ~3u;
     const uint32_t c0 = threadIdx.x * per;
-    uint32_t v[16], sum = 0;
+    uint4 v4[4];
+    uint32_t* const v = (uint32_t*)v4;
+    uint32_t sum = 0;
 #pragma unroll
-    for (uint32_t j = 0; j < 16; ++j) {
-        v[j] = (j < per && c0 + j < C) ? count[c0 + j] : 0u;
-        sum += v[j];
+    for (uint32_t j = 0; j < 16; j += 4) {
+        v4[j / 4] = make_uint4(0u, 0u, 0u, 0u);
+        if (j < per && c0 + j + 4u <= C) {
+            v4[j / 4] = *(const uint4*)(count + c0 + j);
+        } else if (j < per) {
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) v[j + u] = c0 + j + u < C ? count[c0 + j + u] : 0u;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) sum += v[j + u];
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint32_t inc = sum;
@@ -235,12 +248,25 @@ __device__ __forceinline__ void scan_one(uint32_t C, uint32_t* __restrict__ coun
         total += lds[w];
     }
 #pragma unroll
-    for (uint32_t j = 0; j < 16; ++j) {
-        if (j < per && c0 + j < C) {
-            start[c0 + j] = off;
-            count[c0 + j] = 0u;
+    for (uint32_t j = 0; j < 16; j += 4) {
+        uint4 o;
+        o.x = off;
+        o.y = o.x + v[j];
+        o.z = o.y + v[j + 1];
+        o.w = o.z + v[j + 2];
+        off = o.w + v[j + 3];
+        if (j < per && c0 + j + 4u <= C) {
+            *(uint4*)(start + c0 + j) = o;
+            *(uint4*)(count + c0 + j) = make_uint4(0u, 0u, 0u, 0u);
+        } else if (j < per) {
+            const uint32_t w[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+                if (c0 + j + u < C) {
+                    start[c0 + j + u] = w[u];
+                    count[c0 + j + u] = 0u;
+                }
         }
-        off += v[j];
     }
     if (threadIdx.x == 0) start[C] = total;
     if (n == 0) return;
