@@ -1282,7 +1282,7 @@ static void find_knn(gs_group A, gs_knn out, gs_bins bins, gs_group B, uint32_t 
         !split && !(flags & GS_KNN_BINNED) && prefer_exhaustive(B, bins->g, bins->cells, max_distance);
     if ((split || exhaustive) && out->k <= kChunkMaxK && B->n <= kChunkMax) {
         const Seed sd = seed_for(out, A, B, flags);
-        launch_knn_chunks(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map);
+        launch_knn_chunks(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map, split ? std::max(search_radius, 1u) : 0u);
     } else if (split) {
         const Seed sd = seed_for(out, A, B, flags);
         launch_knn_split(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map);

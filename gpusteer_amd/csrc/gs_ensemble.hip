@@ -689,8 +689,8 @@ static void ens_search(gs_ensemble_s* e, const EnsKnnOut& out, int lanes, hipStr
 // at their goals; one lane per query then leaves the step waiting for the few
 // wavefronts whose queries scan thousands of agents of a cell each, so teams
 // pay up to larger sizes than for a flock: 24 scenarios of 220,000 agents over
-// 400 steps 1.03 - 1.19 -> 0.36 ms per step; 64 scenarios of 384,000 agents 0.22 ->
-// 0.27 ms while they are spread out and 0.69 -> 0.35 after 160 steps (left
+// 400 steps 1.03 - 1.19 -> 0.23 ms per step; 64 scenarios of 384,000 agents 0.21 ->
+// 0.25 ms while they are spread out and 0.67 -> 0.29 after 160 steps (left
 // with one lane: the first steps would be slower).
 constexpr uint32_t kTeamMaxCrowds = 262144;
 static int step_lanes(const gs_ensemble_s* e) {

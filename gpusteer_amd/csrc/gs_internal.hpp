@@ -504,10 +504,11 @@ constexpr uint32_t kExhaustiveMax = 4096;
 constexpr uint32_t kSparseCells = 16;
 // A small query group's search of another small group (at most kSplitMaxA
 // queries, at most kSplitMaxPairs query-candidate pairs, B at most
-// kSplitMaxB points) whose reach covers more than kSplitMinCells cells is
-// done by the split exhaustive scan: B cut into ranges of at least
-// kSplitMinRange points, about kSplitWaves wavefronts in all, at most 64
-// ranges.
+// kSplitMaxB points) whose reach covers more than kSplitMinCells cells takes
+// the cells around the query, then B's chunks (launch_knn_chunks with a local
+// radius); lists longer than kChunkMaxK the split exhaustive scan: B cut into
+// ranges of at least kSplitMinRange points, about kSplitWaves wavefronts in
+// all, at most 64 ranges.
 constexpr uint32_t kSplitMaxA = 16384;
 constexpr uint32_t kSplitMaxB = 16384;
 constexpr uint64_t kSplitMaxPairs = 1ull << 26;
@@ -519,11 +520,12 @@ constexpr int kSplitBuf = 16;  // deferred entries per lane
 // chunks beyond the query's bound; lists of up to kChunkMaxK.
 constexpr uint32_t kChunkMax = 16384;
 constexpr uint32_t kChunkMaxK = 16;
-// Words of cbox for n points: min x, y, z, max x, y, z and the points that are
-// numbers, per chunk.
-constexpr size_t chunk_words(uint32_t n) { return 7 * (((size_t)n + 63) / 64); }
+// Words of cbox for n points: min x, y, z, max x, y, z per chunk.
+constexpr size_t chunk_words(uint32_t n) { return 6 * (((size_t)n + 63) / 64); }
+// local: 0, or the cell radius of the box around the query that is searched
+// first (of B's lattice; at most kSplitMaxA queries).
 void launch_knn_chunks(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, const uint32_t* seed,
-                       const uint32_t* row_map, const uint32_t* val_map);
+                       const uint32_t* row_map, const uint32_t* val_map, uint32_t local);
 // The chunk boxes of B's snapshot, if they are not the current one's.
 void launch_chunk_boxes(gs_group_s* B);
 // Whether this thread records a frame (its kernels run at the replays, so

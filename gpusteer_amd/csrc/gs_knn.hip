@@ -175,9 +175,7 @@ void launch_knn_snap_brute(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float ca
 #define GS_SB(KM)                                                                                             \
     k_knn_snap_brute<KM><<<blocks_for(nA), kBlock, 0, st>>>(nA, A->spos.p, B->n, B->spos.p, self, out->k, cap2, \
                                                             out->idx_alt(), out->dist_alt())
-    if (out->k <= 8) GS_SB(8);
-    else if (out->k <= 16) GS_SB(16);
-    else GS_SB(32);
+    GS_SB(32);  // lists of up to kChunkMaxK take launch_knn_chunks
 #undef GS_SB
     GS_LAUNCHED("k_knn_snap_brute");
 }

@@ -1,6 +1,8 @@
-// Exhaustive exact search of small or sparse target groups (walls, obstacles,
-// a small group's search of another far away) by teams of lanes over the
-// target's 64-slot chunks (gs_knn_chunks.hpp).
+// Exact search of small or sparse target groups (walls, obstacles) and of small
+// groups by small groups, by teams of lanes over the target's 64-slot chunks
+// (gs_knn_chunks.hpp).
+#include <cmath>
+
 #include "gs_knn_chunks.hpp"
 
 namespace gs {
@@ -15,7 +17,6 @@ __global__ __launch_bounds__(kBlock) void k_chunk_boxes(uint32_t n, uint32_t chu
     // fminf / fmaxf ignore NaN; a chunk without numbers keeps the empty box.
     float lo[3] = {fminf(p.x, INFINITY), fminf(p.y, INFINITY), fminf(p.z, INFINITY)};
     float hi[3] = {fmaxf(p.x, -INFINITY), fmaxf(p.y, -INFINITY), fmaxf(p.z, -INFINITY)};
-    const uint64_t numbers = __ballot(p.x == p.x && p.y == p.y && p.z == p.z);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
 #pragma unroll
@@ -30,7 +31,6 @@ __global__ __launch_bounds__(kBlock) void k_chunk_boxes(uint32_t n, uint32_t chu
         boxes[a * chunks + c] = lo[a];
         boxes[(3 + a) * chunks + c] = hi[a];
     }
-    boxes[6 * chunks + c] = (float)__popcll(numbers);
 }
 
 void launch_chunk_boxes(gs_group_s* B) {
@@ -41,16 +41,20 @@ void launch_chunk_boxes(gs_group_s* B) {
     B->cbox_fresh = !recording_frame();
 }
 
-template <int G, int KM>
+// Local: the cells around the query first (bstart, g: B's lattice), as far as
+// that takes no more columns than there are chunks; then the chunks.
+template <int G, int KM, int RF, bool Local>
 __global__ __launch_bounds__(kBlock) void k_knn_chunks(uint32_t nA, const float4* __restrict__ apos, uint32_t nB,
                                                        const float4* __restrict__ bpos,
-                                                       const float* __restrict__ boxes, int self, uint32_t k, float cap2,
-                                                       const uint32_t* __restrict__ seed,
+                                                       const float* __restrict__ boxes,
+                                                       const uint32_t* __restrict__ bstart, GridDev g,
+                                                       const uint32_t* __restrict__ box, int self, uint32_t k,
+                                                       float cap2, const uint32_t* __restrict__ seed,
                                                        const uint32_t* __restrict__ row_map,
                                                        const uint32_t* __restrict__ val_map,
                                                        uint32_t* __restrict__ out_idx, float* __restrict__ out_dist) {
-    __shared__ TeamLds<G, KM, 1> lds;
-    TeamList<G, KM, 1> L(lds, k);
+    __shared__ TeamLds<G, KM, RF> lds;
+    TeamList<G, KM, RF> L(lds, k);
     const uint32_t s = blockIdx.x * team_queries<G>() + threadIdx.x / G;
     const bool active = s < nA;
     const float4 q = active ? apos[s] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -59,26 +63,50 @@ __global__ __launch_bounds__(kBlock) void k_knn_chunks(uint32_t nA, const float4
         if (seed)
             thr = fminf(cap2, team_seed_bound(L, active, seed, nA, (active && row_map) ? row_map[s] : s, nB, val_map, q.x,
                                               q.y, q.z, bpos));
-        const FlatQuery Q{q.x, q.y, q.z, thr, self ? s : UINT32_MAX, active};
-        knn_chunks_team(L, Q, nB, bpos, boxes);
+        // As k_knn_binned: no candidate within the cap of B's bounding box.
+        if (box && active && box_beyond(box, q.x, q.y, q.z, cap2)) thr = -1.f;
+        FlatQuery Q{q.x, q.y, q.z, thr, self ? s : UINT32_MAX, active};
+        bool found = false;
+        if (Local) {
+            found = knn_search_team(L, Q, g, nB, bpos, bstart, (int)((nB + 63u) / 64u));
+            Q.thr = L.lim;
+        }
+        if (!found) knn_chunks_team(L, Q, Q.thr == (Local ? cap2 : INFINITY), nB, bpos, boxes);
     }
     if (active) L.store(nA, s, out_idx, out_dist);
 }
 
+// Bound by latency at a few thousand queries, by VALU issue beyond.  131,072
+// agents x 1,254 walls (k = 3, cap 140): 46.5 -> 14.8 us (one lane per query,
+// no seed, before).  Two groups of 5,000 (k = 7, cap of ten cells, a lattice of
+// 120^3): 47 us by ranges per block and a merge, 50 over the chunks alone (a
+// chunk in cell order spans the lattice's depth, and one query without a
+// seed under a wide cap holds its block up), 16 + 3 with the cells around the
+// query first and rings without an end, 20 + 3 here.  The end is at as many
+// columns as chunks: with 5,000 queries of 5,000 points (k = 7, 32^3 cells)
+// mixed / apart / about one cluster, seeded, cap of ten cells: chunks alone 15
+// / 5 / 15 us, no end 20 / 59 / 125, here 27 / 11 / 24; unseeded 71 / 4 / 205,
+// 28 / 58 / 230 and 51 / 11 / 84.
 void launch_knn_chunks(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, const uint32_t* seed,
-                       const uint32_t* row_map, const uint32_t* val_map) {
+                       const uint32_t* row_map, const uint32_t* val_map, uint32_t local) {
     const uint32_t nA = A->n;
     if (nA == 0) return;
     launch_chunk_boxes(B);
     const bool wide = team_lanes(nA, out->k) == 16;
-#define GS_CHUNKS(G, KM)                                                                                       \
-    k_knn_chunks<G, KM><<<blocks_for(nA, team_queries<G>()), kBlock, 0, A->ctx->stream>>>(                     \
-        nA, A->spos.p, B->n, B->spos.p, B->cbox.p, A == B ? 1 : 0, out->k, cap2, seed, row_map, val_map,       \
-        out->idx_alt(), out->dist_alt())
-    if (wide && out->k <= 8) GS_CHUNKS(16, 8);
-    else if (wide) GS_CHUNKS(16, 16);
-    else if (out->k <= 8) GS_CHUNKS(8, 8);
-    else GS_CHUNKS(8, 16);
+    const uint32_t* box = (local && std::isfinite(cap2) && B->bbox_fresh) ? B->bbox[B->bbox_cur].p : nullptr;
+#define GS_CHUNKS(G, KM, RF, Local)                                                                            \
+    k_knn_chunks<G, KM, RF, Local><<<blocks_for(nA, team_queries<G>()), kBlock, 0, A->ctx->stream>>>(          \
+        nA, A->spos.p, B->n, B->spos.p, B->cbox.p, B->start.p, B->bin_grid, box, A == B ? 1 : 0, out->k, cap2, \
+        seed, row_map, val_map, out->idx_alt(), out->dist_alt())
+    static_assert(kSplitMaxA <= kTeam16Max, "a local search has 16 lanes per query");
+    if (local >= 2 && out->k <= 8) GS_CHUNKS(16, 8, 2, true);
+    else if (local >= 2) GS_CHUNKS(16, 16, 2, true);
+    else if (local && out->k <= 8) GS_CHUNKS(16, 8, 1, true);
+    else if (local) GS_CHUNKS(16, 16, 1, true);
+    else if (wide && out->k <= 8) GS_CHUNKS(16, 8, 1, false);
+    else if (wide) GS_CHUNKS(16, 16, 1, false);
+    else if (out->k <= 8) GS_CHUNKS(8, 8, 1, false);
+    else GS_CHUNKS(8, 16, 1, false);
 #undef GS_CHUNKS
     GS_LAUNCHED("k_knn_chunks");
 }

@@ -9,11 +9,26 @@
 
 namespace gs {
 
-// boxes: [7][chunks] (launch_chunk_boxes).  Q as for knn_search_team (thr: the
-// cap or the seed's bound).  Without a bound the nearest chunk that holds
-// enough points gives one: its farthest corner.
+// A lower bound on the d2 of chunk c's points (0 for a query that is no number).
+__device__ __forceinline__ float chunk_gap2(const float* __restrict__ boxes, uint32_t chunks, uint32_t c,
+                                            const float (&q)[3]) {
+    float g2[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float gap = fmaxf(fmaxf(boxes[a * chunks + c] - q[a], q[a] - boxes[(3 + a) * chunks + c]), 0.f);
+        g2[a] = gap * gap;
+    }
+    return (g2[0] + g2[1]) + g2[2];
+}
+
+// boxes: [6][chunks] (launch_chunk_boxes).  Q as for knn_search_team (thr: the
+// cap, a seed's bound or that of a search that gave up).  bound_first: the
+// k-th distance within the nearest chunk bounds the search before it starts;
+// without it a wide bound lets most points of a group into the buffer (5,000
+// queries of 5,000 points about one cluster, k = 7, unseeded, no cap: 96 ->
+// 68 us; 131,072 of 1,254 mixed: 308 -> 116 us).
 template <int G, int KM, int RF>
-__device__ __forceinline__ void knn_chunks_team(TeamList<G, KM, RF>& L, const FlatQuery& Q, uint32_t nB,
+__device__ __forceinline__ void knn_chunks_team(TeamList<G, KM, RF>& L, const FlatQuery& Q, bool bound_first, uint32_t nB,
                                                 const float4* __restrict__ bpos, const float* __restrict__ boxes) {
     const __amdgpu_buffer_rsrc_t rb = pos_rsrc(bpos, nB);
     const uint32_t chunks = (nB + 63u) / 64u;
@@ -21,35 +36,29 @@ __device__ __forceinline__ void knn_chunks_team(TeamList<G, KM, RF>& L, const Fl
     L.cnt = 0;
     L.lim = Q.thr;
     if (!Q.active || Q.thr < 0.f) return;  // the whole team
-    if (L.lim == INFINITY) {
-        float far2 = INFINITY;
+    if (bound_first && chunks > 1u) {
+        float best = INFINITY;
+        uint32_t at = UINT32_MAX;
         for (uint32_t c = L.lane; c < chunks; c += G) {
-            float d2 = 0.f;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const float lo = q[a] - boxes[a * chunks + c], hi = boxes[(3 + a) * chunks + c] - q[a];
-                const float e = fmaxf(fabsf(lo), fabsf(hi));
-                d2 += e * e;
+            const float d2 = chunk_gap2(boxes, chunks, c, q);
+            if (d2 < best) {
+                best = d2;
+                at = c;
             }
-            // more than k points: the query may be one of them
-            if (boxes[6 * chunks + c] > (float)L.k) far2 = fminf(far2, d2 * (1.f + 2e-5f) + 0x1p-100f);
         }
-        // (a NaN distance leaves the bound infinite)
-        L.lim = -L.max_of(-far2);
+        const float near2 = -L.max_of(-best);
+        if (near2 > L.lim) return;  // no chunk in reach
+        if (near2 < INFINITY) {
+            const uint32_t who = L.votes(best == near2);
+            at = (uint32_t)__shfl((int)at, (int)(L.first + (uint32_t)__ffs((int)who) - 1u), 64);
+            int M = 0;
+            L.push_run(at * 64u, L.lane == 0 ? min(64u, nB - at * 64u) : 0u, M);
+            L.lim = fminf(L.lim, L.bound_of(M, Q.x, Q.y, Q.z, Q.self, rb));
+        }
     }
     for (uint32_t c0 = 0; c0 < chunks; c0 += G) {
         const uint32_t c = c0 + L.lane;
-        float d2 = INFINITY;
-        if (c < chunks) {
-            float g2[3];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const float gap =
-                    fmaxf(fmaxf(boxes[a * chunks + c] - q[a], q[a] - boxes[(3 + a) * chunks + c]), 0.f);
-                g2[a] = gap * gap;
-            }
-            d2 = (g2[0] + g2[1]) + g2[2];
-        }
+        const float d2 = c < chunks ? chunk_gap2(boxes, chunks, c, q) : INFINITY;
         int M = 0;
         L.push_run(c * 64u, (c < chunks && d2 <= L.lim) ? min(64u, nB - c * 64u) : 0u, M);
         if (M != 0) L.scan(M, Q.x, Q.y, Q.z, Q.self, rb);

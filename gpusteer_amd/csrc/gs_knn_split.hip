@@ -1,4 +1,5 @@
-// Exact KNN of a small query group by a split exhaustive scan.
+// Exact KNN of a small query group by a split exhaustive scan, for lists longer
+// than kChunkMaxK (shorter ones: gs_knn_chunks.hip).
 //
 // With few queries (a few thousand: the MultiGroup plugin's groups) a
 // one-lane-per-query search runs as a few dozen wavefronts, and a sparse or
@@ -240,10 +241,7 @@ void launch_knn_split(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, c
         launch_knn_snap_brute(A, out, B, cap2);
         return;
     }
-    if (out->k == 7) run_split<7>(A, out, B, cap2, S, seed, row_map, val_map);
-    else if (out->k <= 8) run_split<8>(A, out, B, cap2, S, seed, row_map, val_map);
-    else if (out->k <= 16) run_split<16>(A, out, B, cap2, S, seed, row_map, val_map);
-    else run_split<32>(A, out, B, cap2, S, seed, row_map, val_map);
+    run_split<32>(A, out, B, cap2, S, seed, row_map, val_map);
 }
 
 }  // namespace gs

@@ -278,24 +278,27 @@ __device__ __forceinline__ float team_seed_bound(const TeamList<G, KM, RF>& L, b
 // knn_search_flat; 1 <= nB < kFlatMaxPoints, k <= KM); RF is the first
 // box's column radius (1: 3 x 3, 2: 5 x 5 for lattices finer than the
 // neighbour distance).  Leaves the sorted list in L.  Called by every lane of
-// the wavefront; teams without a query pass active = false.
+// the wavefront; teams without a query pass active = false.  False when the
+// next box would have more than max_columns columns: L.lim is then a bound on
+// the k-th d2 (at most Q.thr) and the list is to be found another way.
 template <int G, int KM, int RF>
-__device__ __forceinline__ void knn_search_team(TeamList<G, KM, RF>& L, const FlatQuery& Q, const GridDev& g,
+__device__ __forceinline__ bool knn_search_team(TeamList<G, KM, RF>& L, const FlatQuery& Q, const GridDev& g,
                                                 uint32_t nB, const float4* __restrict__ bpos,
-                                                const uint32_t* __restrict__ bstart) {
+                                                const uint32_t* __restrict__ bstart, int max_columns = INT_MAX) {
     const __amdgpu_buffer_rsrc_t rb = pos_rsrc(bpos, nB);
     const float grow = 1.0f + 2e-5f;
     const float qx = Q.x, qy = Q.y, qz = Q.z;
     L.cnt = 0;
     L.lim = Q.thr;
-    if (!Q.active || Q.thr < 0.f) return;  // the whole team
+    if (!Q.active || Q.thr < 0.f) return true;  // the whole team
     const int cx = axis_cell_bound(qx, g.ox, g.rx, g.dx);
     const int cy = axis_cell_bound(qy, g.oy, g.ry, g.dy);
     const int cz = axis_cell_bound(qz, g.oz, g.rz, g.dz);
-    // First the box of ring RF, one run per column; then the rings beyond it,
-    // a column per lane and round: a column on the ring's edge in x or y is
-    // one run, the others the two runs above and below the box before.
-    int R = RF, M = 0;
+    // First the box of ring RF, one run per column; then larger boxes (R cells
+    // each way in x and y, R * zr in z), a column per lane and round: a column
+    // outside the box before (ring Rin) is one run, the others the two runs
+    // above and below it.
+    int R = RF, Rin = RF, M = 0;
     // Without a seed or a cap the box is walked twice: for a bound, then for
     // the candidates within it.
     for (bool bound_first = L.lim == INFINITY && L.k <= 2u * G;; bound_first = false) {
@@ -319,7 +322,7 @@ __device__ __forceinline__ void knn_search_team(TeamList<G, KM, RF>& L, const Fl
         if (!bound_first) break;
         L.lim = L.bound_of(M, qx, qy, qz, Q.self, rb);
     }
-    int x0 = 0, y0 = 0, ny = 1, c0 = 0, columns = 0;
+    int c0 = 0, columns = 0;
     bool last = false;  // nothing is left to scan after the runs at hand
     for (;;) {
         L.scan(M, qx, qy, qz, Q.self, rb);
@@ -328,8 +331,22 @@ __device__ __forceinline__ void knn_search_team(TeamList<G, KM, RF>& L, const Fl
             L.reduce();
             bool all;
             const float dmin = outside_gap(g, cx, cy, cz, R, qx, qy, qz, all);
-            if (last || all || exact_after(L.lim, dmin)) return;
-            ++R;
+            if (last || all || exact_after(L.lim, dmin)) return true;
+            // One ring more, then boxes of twice the extent, as far as the
+            // bound reaches: a target far away or a cap without k points
+            // under it is reached in a few rounds.  Ring by ring every step
+            // was a test, a reduction and two dependent loads (a step of 24
+            // scenarios, 220,000 agents: 0.32 -> 0.23 ms).
+            Rin = R;
+            R = R == RF ? R + 1 : 2 * R;
+            if (Rin != RF && L.lim < INFINITY) {
+                float h = INFINITY;
+                if (g.dx > 1) h = fminf(h, g.hx);
+                if (g.dy > 1) h = fminf(h, g.hy);
+                if (g.dz > 1) h = fminf(h, g.hz * (float)g.zr);
+                const float need = (__builtin_amdgcn_sqrtf(L.lim) * grow + g.slack) * __builtin_amdgcn_rcpf(h);
+                if (need < (float)R) R = max(Rin + 1, (int)need + 1);
+            }
             const uint32_t tlo = bstart[0], thi = bstart[(uint32_t)g.dx * (uint32_t)g.dy * (uint32_t)g.dz];
             if (box_beyond_points(g, R, thi - tlo)) {
                 // More cells than points: every point again, the list's own
@@ -339,18 +356,17 @@ __device__ __forceinline__ void knn_search_team(TeamList<G, KM, RF>& L, const Fl
                 L.push_run(tlo, L.lane == 0 ? thi - tlo : 0u, M);
                 continue;
             }
-            x0 = max(cx - R, 0);
-            y0 = max(cy - R, 0);
-            ny = min(cy + R, g.dy - 1) - y0 + 1;
-            columns = (min(cx + R, g.dx - 1) - x0 + 1) * ny;
+            columns = (min(cx + R, g.dx - 1) - max(cx - R, 0) + 1) * (min(cy + R, g.dy - 1) - max(cy - R, 0) + 1);
+            if (columns > max_columns) return false;
             c0 = 0;
         }
-        const int Z = R * g.zr, Zin = (R - 1) * g.zr;
+        const int Z = R * g.zr, Zin = Rin * g.zr;
+        const int x0 = max(cx - R, 0), y0 = max(cy - R, 0), ny = min(cy + R, g.dy - 1) - y0 + 1;
         for (; M == 0 && c0 < columns; c0 += G) {
             const int c = c0 + (int)L.lane;
             const int ix = x0 + c / ny, iy = y0 + c % ny;
             const bool valid = c < columns;
-            const bool edge = ix == cx - R || ix == cx + R || iy == cy - R || iy == cy + R;
+            const bool edge = abs(ix - cx) > Rin || abs(iy - cy) > Rin;
             const float gx = axis_gap(qx, ix, ix, g.ox, g.hx, g.dx, g.slack);
             const float gy = axis_gap(qy, iy, iy, g.oy, g.hy, g.dy, g.slack);
             const float gxy = gx * gx + gy * gy;

@@ -67,6 +67,42 @@ def test_lists(gs, ctx, orc, na, nb, k, cells, cap):
     _check(gs, ctx, orc, _points(na, na), _points(nb, nb + 1) if nb else None, k, cells, cap)
 
 
+# Small groups by small groups: the cells around the query, wider boxes while
+# they have no more columns than the target has chunks, then the chunks.
+@pytest.mark.parametrize("where", ["mixed", "apart", "one cluster"])
+@pytest.mark.parametrize("na,nb,k,radius,cap", [
+    (2000, 1025, 1, 1, 40.0), (2000, 1025, 7, 2, 75.0), (1999, 4096, 8, 1, None), (513, 1024, 9, 2, 1e6),
+    (300, 10000, 16, 1, 60.0), (16384, 257, 7, 1, None)])
+def test_small_groups(gs, ctx, orc, where, na, nb, k, radius, cap):
+    print(f"case {where} na={na} nb={nb} k={k} radius={radius} cap={cap}", flush=True)
+    g = np.random.default_rng(na + nb)
+    lo, hi = {"mixed": (-100.0, 100.0), "apart": (60.0, 100.0), "one cluster": (-8.0, 8.0)}[where]
+    a = g.uniform(-100.0, -60.0 if where == "apart" else 100.0, (na, 3)).astype(np.float32)
+    b = g.uniform(lo, hi, (nb, 3)).astype(np.float32)
+    bins = gs.KNNBinData(ctx, (23, 20, 24), (200.0, 200.0, 200.0))
+    A, B = _group(gs, ctx, a), _group(gs, ctx, b)
+    knn = gs.KNNData(ctx, na, k)
+    limit = float("inf") if cap is None else cap
+    for step in range(3):
+        if step != 1:
+            for G in (A, B):
+                gs.updateKNNDatabase(G, bins)
+        if cap is None:
+            gs.findKNearestNeighbors(A, knn, bins, B, radius)
+        else:
+            gs.findKNearestNeighborsWithin(A, knn, bins, B, cap, radius)
+        idx, dist = knn.download()
+        q = np.unique(np.linspace(0, na - 1, 300).astype(np.uint32))
+        r_idx, r_dist = orc.knn_brute(A.download().pos(), B.download().pos(), k, False, queries=q, cap=limit)
+        np.testing.assert_array_equal(idx[:, q], r_idx[:, q])
+        np.testing.assert_array_equal(dist[:, q], r_dist[:, q])
+        if step == 1:  # part of each group goes to the opposite face: seeds far away
+            for G in (A, B):
+                gs.wrapWorld(G, worldSize=(150.0, 150.0, 150.0))
+    for h in (knn, bins, A, B):
+        h.close()
+
+
 def test_far_targets_and_odd_coordinates(gs, ctx, orc):
     a, b = _points(3000, 3), _points(200, 4, spread=5.0) + np.float32([5e4, 0.0, -5e4])
     _check(gs, ctx, orc, a, b, 7, (40, 1, 40), None)
