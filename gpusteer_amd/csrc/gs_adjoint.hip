@@ -239,9 +239,62 @@ __device__ __forceinline__ bool hood(f3 off, float d2, f3 fwd, const FlockTerm& 
     return dot3(fwd, off / d) > t.cos_max;
 }
 
+// The positions of an agent's listed neighbours, read once per kernel into the
+// lane's LDS column: the step walks its two lists seven times (separation,
+// alignment, cohesion, penetration, and in the adjoint twice more), each time a
+// chain of two dependent loads per neighbour, which bounded both kernels.
+// Positions of both lists up to their first pad; k is at most kNb (an
+// ensemble's limit).  131,072 agents, k = 7: forward 29.6 -> 24.3 us, backward
+// 68.4 -> 49.9 us; 48 KB leave three blocks per CU, as many as their registers.
+constexpr int kNb = 8;
+struct Neighbours {
+    float* col;  // [2][kNb][3][kBlock] floats, this lane's column
+    int m[2];    // entries before the first pad: own group, other group
+    __device__ __forceinline__ f3 pos(int w, int j) const {
+        const float* p = col + (w * kNb + j) * 3 * kBlock;
+        return mk3(p[0], p[kBlock], p[2 * kBlock]);
+    }
+};
+#define C4_NEIGHBOURS_LDS __shared__ float lds_nb[2 * kNb * 3 * kBlock];
+__device__ __forceinline__ Neighbours c4_neighbours(const CalibDev& D, uint32_t i, const CState& X,
+                                                    const uint32_t* __restrict__ kself,
+                                                    const uint32_t* __restrict__ kother, float* lds) {
+    Neighbours nb;
+    nb.col = lds + threadIdx.x;
+    uint32_t b[2][kNb];
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int j = 0; j < kNb; ++j)
+            b[w][j] = (w == 0 ? kself : kother)[(size_t)min(j, (int)D.k - 1) * D.N + i];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        nb.m[w] = (int)D.k;
+#pragma unroll
+        for (int j = kNb - 1; j >= 0; --j)
+            if (j < (int)D.k && b[w][j] >= D.N) nb.m[w] = j;
+    }
+    // Unconditional loads (the agent itself past the pad), all in flight.
+    f3 p[2][kNb];
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int j = 0; j < kNb; ++j) p[w][j] = ldS(X, 0, j < nb.m[w] ? b[w][j] : i);
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int j = 0; j < kNb; ++j) {
+            float* q = nb.col + (w * kNb + j) * 3 * kBlock;
+            q[0] = p[w][j].x;
+            q[kBlock] = p[w][j].y;
+            q[2 * kBlock] = p[w][j].z;
+        }
+    return nb;
+}
+
 // One agent's step.  Returns the new state; fills rec.
 __device__ __forceinline__ void c4_fwd_agent(const CalibDev& D, const EnsPop& P, const EnsScen& S, uint32_t i,
-                                             const CState& X, const uint32_t* __restrict__ kself,
+                                             const CState& X, const Neighbours& nb, const uint32_t* __restrict__ kself,
                                              const uint32_t* __restrict__ kother, const uint32_t* __restrict__ kw,
                                              const uint32_t* __restrict__ ko, C4In& in, f3& p1, f3& f1, f3& G,
                                              f3& pn, f3& fn, float& sn, f3& sdn, f3& upn, C4Rec& rec) {
@@ -299,7 +352,6 @@ __device__ __forceinline__ void c4_fwd_agent(const CalibDev& D, const EnsPop& P,
         apply(G, bits, fo, D.th.w_obs[g], GS_BIT_AVOID_OBSTACLES);
     }
     // separation: own group, then the other group
-    const uint32_t* lists[2] = {kself, kother};
     for (int w = 0; w < 2; ++w) {
         uint32_t m = 0u;
         int on = 0;
@@ -307,10 +359,8 @@ __device__ __forceinline__ void c4_fwd_agent(const CalibDev& D, const EnsPop& P,
         int cnt = 0;
         if (!(bits & D.mask_sep)) {
             on = 1;
-            for (uint32_t j = 0; j < D.k; ++j) {
-                const uint32_t b = lists[w][(size_t)j * D.N + i];
-                if (b >= D.N) break;
-                const f3 off = ldS(X, 0, b) - p1;
+            for (int j = 0; j < nb.m[w]; ++j) {
+                const f3 off = nb.pos(w, j) - p1;
                 const float d2 = dot3(off, off);
                 if (hood(off, d2, f1, D.sep)) {
                     acc = acc + off / -d2;
@@ -336,12 +386,10 @@ __device__ __forceinline__ void c4_fwd_agent(const CalibDev& D, const EnsPop& P,
         int cnt = 0;
         rec.on_al = !(bits & D.ali.mask) ? 1 : 0;
         if (rec.on_al) {
-            for (uint32_t j = 0; j < D.k; ++j) {
-                const uint32_t b = kself[(size_t)j * D.N + i];
-                if (b >= D.N) break;
-                const f3 off = ldS(X, 0, b) - p1;
+            for (int j = 0; j < nb.m[0]; ++j) {
+                const f3 off = nb.pos(0, j) - p1;
                 if (hood(off, dot3(off, off), f1, D.ali)) {
-                    acc = acc + ldS(X, 3, b);
+                    acc = acc + ldS(X, 3, kself[(size_t)j * D.N + i]);
                     ++cnt;
                     m |= 1u << j;
                 }
@@ -358,10 +406,8 @@ __device__ __forceinline__ void c4_fwd_agent(const CalibDev& D, const EnsPop& P,
         int cnt = 0;
         rec.on_co = !(bits & D.coh.mask) ? 1 : 0;
         if (rec.on_co) {
-            for (uint32_t j = 0; j < D.k; ++j) {
-                const uint32_t b = kself[(size_t)j * D.N + i];
-                if (b >= D.N) break;
-                const f3 pb = ldS(X, 0, b);
+            for (int j = 0; j < nb.m[0]; ++j) {
+                const f3 pb = nb.pos(0, j);
                 const f3 off = pb - p1;
                 if (hood(off, dot3(off, off), f1, D.coh)) {
                     acc = acc + pb;
@@ -406,17 +452,14 @@ __device__ __forceinline__ uint32_t agent_block_pop(const CalibDev& D, uint32_t 
 // Penetration term of step t for agent i: pairs with its own-group and
 // other-group lists, positions of step t.
 __device__ __forceinline__ float pen_loss(const CalibDev& D, const EnsPop& P, uint32_t i, const CState& X,
-                                          const uint32_t* __restrict__ kself, const uint32_t* __restrict__ kother) {
+                                          const Neighbours& nb) {
     const f3 p = ldS(X, 0, i);
     const int g = P.group;
     float L = 0.f;
     for (int w = 0; w < 2; ++w) {
-        const uint32_t* lst = w == 0 ? kself : kother;
         const float R = D.th.radius[g] + D.th.radius[w == 0 ? g : 1 - g];
-        for (uint32_t j = 0; j < D.k; ++j) {
-            const uint32_t b = lst[(size_t)j * D.N + i];
-            if (b >= D.N) break;
-            const float e = R - len3(ldS(X, 0, b) - p);
+        for (int j = 0; j < nb.m[w]; ++j) {
+            const float e = R - len3(nb.pos(w, j) - p);
             if (e > 0.f) L += e * e;
         }
     }
@@ -518,7 +561,15 @@ __global__ __launch_bounds__(kBlock) void c4_rev_rank(uint32_t N, const uint32_t
     const uint32_t s0 = rstart[b], s1 = rstart[b + 1];
     const uint32_t c = rev[s];
     uint32_t r = 0;
-    for (uint32_t t = s0; t < s1; ++t) r += rev[t] < c ? 1u : 0u;
+    // Eight at a time: one dependent load per member before (12.1 -> 11.0 us
+    // for 131,072 agents).
+    for (uint32_t t = s0; t < s1; t += 8) {
+        uint32_t o[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) o[u] = rev[min(t + u, s1 - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) r += (t + u < s1 && o[u] < c) ? 1u : 0u;
+    }
     slot_of[c] = s0 + r;
 }
 
@@ -528,6 +579,7 @@ __global__ __launch_bounds__(kBlock) void c4_forward(CalibDev D, CState X, CStat
                                                      const uint32_t* __restrict__ kw, const uint32_t* __restrict__ ko,
                                                      double* __restrict__ loss_part) {
     __shared__ double lds[kBlock / 64];
+    C4_NEIGHBOURS_LDS
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t i = blk * blockDim.x + threadIdx.x;
     const EnsPop& P = D.pops[D.block_pop[blk]];
@@ -538,13 +590,14 @@ __global__ __launch_bounds__(kBlock) void c4_forward(CalibDev D, CState X, CStat
         C4Rec rec;
         f3 p1, f1, G, pn, fn, sdn, upn;
         float sn;
-        c4_fwd_agent(D, P, S, i, X, kself, kother, kw, ko, in, p1, f1, G, pn, fn, sn, sdn, upn, rec);
+        const Neighbours nb = c4_neighbours(D, i, X, kself, kother, lds_nb);
+        c4_fwd_agent(D, P, S, i, X, nb, kself, kother, kw, ko, in, p1, f1, G, pn, fn, sn, sdn, upn, rec);
         Y.a[0][i] = pn.x; Y.a[1][i] = pn.y; Y.a[2][i] = pn.z;
         Y.a[3][i] = fn.x; Y.a[4][i] = fn.y; Y.a[5][i] = fn.z;
         Y.a[6][i] = sn;
         Y.a[7][i] = sdn.x; Y.a[8][i] = sdn.y; Y.a[9][i] = sdn.z;
         Y.a[10][i] = upn.x; Y.a[11][i] = upn.y; Y.a[12][i] = upn.z;
-        lp = pen_loss(D, P, i, X, kself, kother) * D.inv_S;
+        lp = pen_loss(D, P, i, X, nb) * D.inv_S;
     }
     if (loss_part) block_add(lp, loss_part + blockIdx.x, lds);
 }
@@ -594,6 +647,7 @@ __global__ __launch_bounds__(kBlock) void c4_backward(CalibDev D, CState X, cons
                                                       float4* __restrict__ contrib_out,
                                                       double* __restrict__ grad_part) {
     __shared__ double lds[kBlock / 64];
+    C4_NEIGHBOURS_LDS
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t i = blk * blockDim.x + threadIdx.x;
     const EnsPop& P = D.pops[D.block_pop[blk]];
@@ -607,11 +661,13 @@ __global__ __launch_bounds__(kBlock) void c4_backward(CalibDev D, CState X, cons
         C4Rec rec;
         f3 p1, f1, G, pn, fn, sdn, upn;
         float sn;
-        c4_fwd_agent(D, P, S, i, X, kself, kother, kw, ko, in, p1, f1, G, pn, fn, sn, sdn, upn, rec);
+        const Neighbours nb = c4_neighbours(D, i, X, kself, kother, lds_nb);
+        c4_fwd_agent(D, P, S, i, X, nb, kself, kother, kw, ko, in, p1, f1, G, pn, fn, sn, sdn, upn, rec);
         // neighbour terms of the step after, in segment order
         f3 accp = mk3(0.f, 0.f, 0.f), accf = accp;
         if (rstart_in) {
             const uint32_t s1 = rstart_in[i + 1];
+#pragma unroll 4
             for (uint32_t s = rstart_in[i]; s < s1; ++s) {
                 const float4 u = contrib_in[2 * (size_t)s], v = contrib_in[2 * (size_t)s + 1];
                 accp = accp + mk3(u.x, u.y, u.z);
@@ -660,24 +716,20 @@ __global__ __launch_bounds__(kBlock) void c4_backward(CalibDev D, CState X, cons
         f3 nb_coh = mk3(0.f, 0.f, 0.f), nb_ali = nb_coh, ab_ss = nb_coh, ab_so = nb_coh;
         {
             f3 sc = mk3(0.f, 0.f, 0.f), sa = sc, s_ss = sc, s_so = sc;
-            for (uint32_t j = 0; j < D.k; ++j) {
-                const uint32_t b = kself[(size_t)j * D.N + i];
-                if (b >= D.N) break;
+            for (int j = 0; j < nb.m[0]; ++j) {
                 const uint32_t bit = 1u << j;
                 if (!((rec.m_co | rec.m_al | rec.m_ss) & bit)) continue;
-                const f3 pj = ldS(X, 0, b);
+                const f3 pj = nb.pos(0, j);
                 if (rec.m_co & bit) sc = sc + pj;
-                if (rec.m_al & bit) sa = sa + ldS(X, 3, b);
+                if (rec.m_al & bit) sa = sa + ldS(X, 3, kself[(size_t)j * D.N + i]);
                 if (rec.m_ss & bit) {
                     const f3 off = pj - p1;
                     s_ss = s_ss + off / -dot3(off, off);
                 }
             }
-            for (uint32_t j = 0; j < D.k; ++j) {
-                const uint32_t b = kother[(size_t)j * D.N + i];
-                if (b >= D.N) break;
+            for (int j = 0; j < nb.m[1]; ++j) {
                 if (rec.m_so & (1u << j)) {
-                    const f3 off = ldS(X, 0, b) - p1;
+                    const f3 off = nb.pos(1, j) - p1;
                     s_so = s_so + off / -dot3(off, off);
                 }
             }
@@ -713,16 +765,16 @@ __global__ __launch_bounds__(kBlock) void c4_backward(CalibDev D, CState X, cons
         // ---- per-neighbour pass: separation, cohesion, alignment and the
         // step's penetration term, one accumulation per neighbour slot
         for (int w = 0; w < 2; ++w) {
-            const uint32_t* lst = w == 0 ? kself : kother;
             const uint32_t msep = w == 0 ? rec.m_ss : rec.m_so;
             const f3 ab = w == 0 ? ab_ss : ab_so;
             const int go = w == 0 ? g : 1 - g;
             const float R = D.th.radius[g] + D.th.radius[go];
-            for (uint32_t j = 0; j < D.k; ++j) {
-                const uint32_t b = lst[(size_t)j * D.N + i];
-                if (b >= D.N) break;
+            uint32_t slot = slot_out[rev_code(i, (uint32_t)w, 0u, D.k)];  // read one entry ahead
+            for (int j = 0; j < nb.m[w]; ++j) {
+                const size_t so = slot;
+                if (j + 1 < nb.m[w]) slot = slot_out[rev_code(i, (uint32_t)w, (uint32_t)j + 1u, D.k)];
                 const uint32_t bit = 1u << j;
-                const f3 pj = ldS(X, 0, b);
+                const f3 pj = nb.pos(w, j);
                 f3 cp = mk3(0.f, 0.f, 0.f), cf = cp;
                 if (msep & bit) {
                     const f3 off = pj - p1;
@@ -747,7 +799,6 @@ __global__ __launch_bounds__(kBlock) void c4_backward(CalibDev D, CState X, cons
                     cp = cp + gpj;
                     pb = pb - gpj;
                 }
-                const size_t so = slot_out[rev_code(i, (uint32_t)w, j, D.k)];
                 contrib_out[2 * so] = make_float4(cp.x, cp.y, cp.z, cf.x);
                 contrib_out[2 * so + 1] = make_float4(cf.y, cf.z, 0.f, 0.f);
             }

@@ -235,3 +235,35 @@ def test_calibration_workload_100_steps_vs_tangent(ctx, orc):
     ok = _rel_ok(grad, t32, 1e-3)
     assert ok.all(), f"components {np.nonzero(~ok)[0]}: gpu {grad[~ok]} tangent {t32[~ok]}"
     assert _rel_ok(grad2, grad, 1e-4).all()
+
+
+@pytest.mark.parametrize("n,k", [(200, 1), (200, 8), (10, 7), (12, 8)])
+def test_list_lengths(ctx, orc, n, k):
+    """The shortest and longest lists, and groups with fewer neighbours than
+    list slots (5 and 6 agents a side): state bit for bit, gradient within the
+    bounds of test_adjoint_matches_finite_differences."""
+    cfg = scenarios.CalibConfig(steps=5, checkpoint_every=2)
+    sc = scenarios.choke(n_total=n, workload=21)
+    sc.mode = 1
+    th = scenarios.calib_params()
+    ens = Ensemble(ctx, [("choke", sc)], k=k)
+    cal = Calibration(ens, cfg)
+    loss = cal.forward(th)
+    grad = cal.backward()
+    c = orc.C4(sc, cfg, k)
+    _, fs32 = c.run(th, 1, want_state=True, precision=32)
+    n0, n1 = sc.groups[0].n, sc.groups[1].n
+    for g, (off, m) in enumerate(((0, n0), (13 * n0, n1))):
+        gpu = cal.final_state(0, g)
+        for j, f in enumerate(orc.C4_STATE):
+            np.testing.assert_array_equal(gpu.arrays[f], fs32[off + j * m: off + (j + 1) * m].astype(np.float32),
+                                          err_msg=f"group {g} field {f}")
+    base, fd = c.fd_grad(th, 1e-4, record_precision=32)
+    c.close()
+    print("grad gpu", np.array2string(grad, precision=5))
+    print("grad fd ", np.array2string(fd, precision=5), flush=True)
+    assert abs(loss - base) <= 1e-5 * abs(base)
+    bad = np.abs(grad - fd) > 1e-3 * np.abs(fd) + 1e-6 * np.max(np.abs(fd))
+    assert not bad.any(), f"components {np.nonzero(bad)[0]}: gpu {grad[bad]} fd {fd[bad]}"
+    cal.close()
+    ens.close()
