@@ -78,10 +78,10 @@ __global__ __launch_bounds__(kBlock) void k_knn_chunks(uint32_t nA, const float4
 
 // Bound by latency at a few thousand queries, by VALU issue beyond.  131,072
 // agents x 1,254 walls (k = 3, cap 140): 46.5 -> 14.8 us (one lane per query,
-// no seed, before).  Two groups of 5,000 (k = 7, cap of ten cells, a lattice of
-// 120^3): 47 us by ranges per block and a merge, 50 over the chunks alone (a
-// chunk in cell order spans the lattice's depth, and one query without a
-// seed under a wide cap holds its block up), 16 + 3 with the cells around the
+// no seed, before).  Two groups of 5,000 (k = 7, cap of ten cells, 100 x 1 x
+// 100 cells): 47 us by ranges per block and a merge, 50 over the chunks alone (a
+// chunk is a strip across the lattice, and one query without a seed under a
+// wide cap holds its block up), 16 + 3 with the cells around the
 // query first and rings without an end, 20 + 3 here.  The end is at as many
 // columns as chunks: with 5,000 queries of 5,000 points (k = 7, 32^3 cells)
 // mixed / apart / about one cluster, seeded, cap of ten cells: chunks alone 15

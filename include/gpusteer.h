@@ -235,8 +235,9 @@ int gs_update_knn_database(gs_group g, gs_bins bins);
  * for the same A, B and memberships bounds the search (result unchanged).
  * Unless GS_KNN_BINNED, a small A searching another small group B (at most
  * 16384 agents each, at most 2^26 pairs) over more than 64 cells of reach is
- * served by an exhaustive scan of B's snapshot split over many wavefronts,
- * and a small or sparse B by an exhaustive scan: the same exact result. */
+ * served by the cells around each query and then by B's snapshot in chunks
+ * (k > 16: by a scan split over many wavefronts), and a small or sparse B by
+ * its chunks alone: the same exact result. */
 int gs_find_knn(gs_group A, gs_knn out, gs_bins bins, gs_group B, uint32_t search_radius, uint32_t flags);
 /* gs_find_knn restricted to points closer than max_distance (strict, the
  * locality test of src/lq.c:327: d^2 < r^2 in fp32); rows with fewer than k
