@@ -481,7 +481,7 @@ void launch_scatter_reorder(uint32_t n, const uint32_t* key, const uint32_t* ran
         k_scatter<<<blocks_for(n), kBlock, 0, st>>>(n, key, rank, start, ids, id_tmp);
         GS_LAUNCHED("k_scatter");
     }
-    k_reorder<<<blocks_for(n), kBlock, 0, st>>>(n, rank, id_tmp, key, start, ids, ids_new, new_to_old,
+    k_reorder<<<agent_blocks(n), agent_block(n), 0, st>>>(n, rank, id_tmp, key, start, ids, ids_new, new_to_old,
                                                 old_to_new, bits, bits_new, fs, spos, sfwd);
     GS_LAUNCHED("k_reorder");
 }
@@ -580,7 +580,7 @@ void launch_pair_build(gs_group_s* const g[2], const gs_bins_s* b) {
     GS_LAUNCHED("k_pair_key");
     k_pair_scan<<<dim3(1, 2), kScanOneThreads, 0, st>>>(P, b->cells);
     GS_LAUNCHED("k_pair_scan");
-    k_pair_reorder<<<dim3(blocks_for(n), 2), kBlock, 0, st>>>(P);
+    k_pair_reorder<<<dim3(agent_blocks(n), 2), agent_block(n), 0, st>>>(P);
     GS_LAUNCHED("k_pair_reorder");
     for (int i = 0; i < 2; ++i) end_build(g[i], moved[i], bits[i]);
 }

@@ -55,6 +55,16 @@ void hip_check(hipError_t e, const char* what);
 
 constexpr int kBlock = 256;
 inline unsigned blocks_for(uint64_t n, unsigned per = kBlock) { return (unsigned)((n + per - 1) / per); }
+// Threads per block of a kernel with one lane per agent and nothing shared in
+// its blocks: one wavefront for small groups, so that they lie on four times
+// as many CUs (the kernels gather, and a CU serves one wavefront's scattered
+// loads after the other).  Blocks of 256 / 64 threads, us: fused step, 4,096
+// agents 30.1 / 28.8, 16,384 29.9 / 29.1, 32,768 37.9 / 37.5, 65,536 43.2 /
+// 44.1, 131,072 56.5 / 57.3; two behaviours and an integrate by separate calls,
+// 16,384 16.8 / 14.5, 32,768 17.0 / 16.4, 65,536 19.0 / 19.2.
+constexpr uint32_t kSmallBlocksMax = 32768;
+inline unsigned agent_block(uint64_t n) { return n <= kSmallBlocksMax ? 64u : (unsigned)kBlock; }
+inline unsigned agent_blocks(uint64_t n) { return blocks_for(n, agent_block(n)); }
 
 // ---------------------------------------------------------------------------
 // Device memory: a typed buffer that grows on demand.  Owned by handles.

@@ -161,7 +161,8 @@ static void run_flock(gs_group_s* A, gs_knn_s* knn, gs_group_s* B, const gs_floc
     hipStream_t st = A->ctx->stream;
     const Agents a = A->dev_agents();
 #define GS_FLOCK(MODE)                                                                                              \
-    k_flock<KMAX, MODE><<<blocks_for(A->n), kBlock, 0, st>>>(A->n, a, B->n, B->F(0), B->F(1), B->F(2), B->F(3),      \
+    k_flock<KMAX, MODE><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(                                         \
+        A->n, a, B->n, B->F(0), B->F(1), B->F(2), B->F(3),                                                         \
                                                              B->F(4), B->F(5), knn->idx(), knn->k, term(sep),        \
                                                              term(ali), term(coh))
     if (mode == GS_MODE_GPUREF) GS_FLOCK(GS_MODE_GPUREF);
@@ -183,9 +184,11 @@ void launch_seek(gs_group_s* A, const float* t, float w, uint32_t mask, int mode
     if (A->n == 0) return;
     hipStream_t st = A->ctx->stream;
     if (mode == GS_MODE_GPUREF)
-        k_seek<GS_MODE_GPUREF><<<blocks_for(A->n), kBlock, 0, st>>>(A->n, A->dev_agents(), t[0], t[1], t[2], w, mask);
+        k_seek<GS_MODE_GPUREF><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(
+            A->n, A->dev_agents(), t[0], t[1], t[2], w, mask);
     else
-        k_seek<GS_MODE_OPENSTEER><<<blocks_for(A->n), kBlock, 0, st>>>(A->n, A->dev_agents(), t[0], t[1], t[2], w,
+        k_seek<GS_MODE_OPENSTEER><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(
+            A->n, A->dev_agents(), t[0], t[1], t[2], w,
                                                                        mask);
     GS_LAUNCHED("k_seek");
     A->mark_written(kFSteer, true);
@@ -193,7 +196,8 @@ void launch_seek(gs_group_s* A, const float* t, float w, uint32_t mask, int mode
 
 void launch_avoid_obstacles(gs_group_s* A, gs_group_s* O, gs_knn_s* knn, float min_time, float w, uint32_t mask) {
     if (A->n == 0) return;
-    k_avoid_obstacles<<<blocks_for(A->n), kBlock, 0, A->ctx->stream>>>(A->n, A->dev_agents(), O->n, O->F(0),
+    k_avoid_obstacles<<<agent_blocks(A->n), agent_block(A->n), 0, A->ctx->stream>>>(
+        A->n, A->dev_agents(), O->n, O->F(0),
                                                                         O->F(1), O->F(2), O->F(19), knn->idx(),
                                                                         knn->k, min_time, w, mask);
     GS_LAUNCHED("k_avoid_obstacles");
@@ -205,7 +209,8 @@ void launch_avoid_walls(gs_group_s* A, gs_knn_s* knn, gs_group_s* W, float min_t
     const int f0 = kWallField;
     gs_walls wd{W->F(f0), W->F(f0 + 1), W->F(f0 + 2), W->F(f0 + 3), W->F(f0 + 4),
                 W->F(f0 + 5), W->F(f0 + 6), W->F(f0 + 7), W->F(f0 + 8)};
-    k_avoid_walls<<<blocks_for(A->n), kBlock, 0, A->ctx->stream>>>(A->n, A->dev_agents(), W->n, wd, knn->idx(),
+    k_avoid_walls<<<agent_blocks(A->n), agent_block(A->n), 0, A->ctx->stream>>>(
+        A->n, A->dev_agents(), W->n, wd, knn->idx(),
                                                                     knn->k, min_time, w, mask);
     GS_LAUNCHED("k_avoid_walls");
     // touching agents are moved and turned (positions, forward vectors)
@@ -216,16 +221,17 @@ void launch_update(gs_group_s* A, float dt, int mode) {
     if (A->n == 0) return;
     hipStream_t st = A->ctx->stream;
     if (mode == GS_MODE_GPUREF)
-        k_update<GS_MODE_GPUREF><<<blocks_for(A->n), kBlock, 0, st>>>(A->n, A->dev_agents(), dt);
+        k_update<GS_MODE_GPUREF><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(A->n, A->dev_agents(), dt);
     else
-        k_update<GS_MODE_OPENSTEER><<<blocks_for(A->n), kBlock, 0, st>>>(A->n, A->dev_agents(), dt);
+        k_update<GS_MODE_OPENSTEER><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(A->n, A->dev_agents(), dt);
     GS_LAUNCHED("k_update");
     A->mark_integrated();
 }
 
 void launch_wrap(gs_group_s* A, int shape, const float* c, const float* s) {
     if (A->n == 0) return;
-    k_wrap<<<blocks_for(A->n), kBlock, 0, A->ctx->stream>>>(A->n, A->F(0), A->F(1), A->F(2), shape, c[0], c[1], c[2],
+    k_wrap<<<agent_blocks(A->n), agent_block(A->n), 0, A->ctx->stream>>>(
+        A->n, A->F(0), A->F(1), A->F(2), shape, c[0], c[1], c[2],
                                                             s[0], s[1], s[2]);
     GS_LAUNCHED("k_wrap");
     A->mark_written(kFPos, false);

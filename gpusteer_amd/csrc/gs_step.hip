@@ -282,7 +282,10 @@ static void run_flock_update(gs_group_s* A, gs_knn_s* knn, const gs_boids_params
         else if (sh.block == 256 && sh.apl == 2) GS_FU(MODE, 256, 2);                                                \
         else if (sh.block == 512 && sh.apl == 1) GS_FU(MODE, 512, 1);                                                \
         else if (sh.block == 512 && sh.apl == 2) GS_FU(MODE, 512, 2);                                                \
+        else if (agent_block(n) == 64u) GS_FU(MODE, 64, 1);                                                          \
         else GS_FU(MODE, kBlock, 1);                                                                                 \
+    } else if (agent_block(n) == 64u) {                                                                              \
+        GS_FU(MODE, 64, 1);                                                                                          \
     } else {                                                                                                         \
         GS_FU(MODE, kBlock, 1);                                                                                      \
     }

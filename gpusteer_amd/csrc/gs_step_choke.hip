@@ -5,8 +5,8 @@
 // cost is launches and latency, on a chip that is nearly empty.  Here a frame
 // is six: the builds' three passes (gs_bins.hip), the eight searches, walls and
 // obstacles, separation with seek and the integrate, each over both groups.
-// 10,000 agents: 159 -> 55 us a frame (search 14.7, reorder 9.9, integrate 8.8,
-// walls and obstacles 7.4, scan 6.7, keys 3.7 us).
+// 10,000 agents: 159 -> 54 us a frame (search 14.2, reorder 9.5, integrate 8.0,
+// walls and obstacles 6.9, scan 6.6, keys 3.8 us).
 //
 // Same results, bit for bit.  Between the calls of the sequence the groups see
 // each other's state: group 0's separation from group 1 reads group 1's
@@ -121,7 +121,7 @@ struct PairSteer {
 __global__ __launch_bounds__(kBlock) void k_pair_avoid(PairSteer P) {
     const PairAgents& G = P.a[blockIdx.y];
     const Agents& A = G.A;
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= G.n) return;
     uint32_t bits = 0u;
     f3 pos = ld3(A.px, A.py, A.pz, i), dir = ld3(A.fx, A.fy, A.fz, i);
@@ -144,7 +144,7 @@ template <int MODE>
 __global__ __launch_bounds__(kBlock) void k_pair_finish(PairSteer P) {
     const PairAgents &G = P.a[blockIdx.y], &H = P.a[1 - blockIdx.y];
     const Agents& A = G.A;
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= G.n) return;
     uint32_t bits = A.bits[i];
     f3 steering = ld3(A.gx, A.gy, A.gz, i);
@@ -217,11 +217,12 @@ void launch_pair_steer(gs_group_s* const g[2], gs_group_s* W, gs_group_s* O, gs_
     const gs_flock_term& t = s->choke_separation;
     P.sep = FlockTerm{t.min_d, t.max_d, t.cos_max, t.weight, t.mask, 1};
     hipStream_t st = g[0]->ctx->stream;
-    const dim3 grid(blocks_for(n), 2);
-    k_pair_avoid<<<grid, kBlock, 0, st>>>(P);
+    const unsigned block = agent_block(n);
+    const dim3 grid(agent_blocks(n), 2);
+    k_pair_avoid<<<grid, block, 0, st>>>(P);
     GS_LAUNCHED("k_pair_avoid");
-    if (s->mode == GS_MODE_GPUREF) k_pair_finish<GS_MODE_GPUREF><<<grid, kBlock, 0, st>>>(P);
-    else k_pair_finish<GS_MODE_OPENSTEER><<<grid, kBlock, 0, st>>>(P);
+    if (s->mode == GS_MODE_GPUREF) k_pair_finish<GS_MODE_GPUREF><<<grid, block, 0, st>>>(P);
+    else k_pair_finish<GS_MODE_OPENSTEER><<<grid, block, 0, st>>>(P);
     GS_LAUNCHED("k_pair_finish");
     for (int i = 0; i < 2; ++i) {
         for (int j = 0; j < 6; ++j) g[i]->flip(j);
