@@ -168,14 +168,20 @@ struct Transfer {
     std::unique_lock<std::mutex> lock;
     explicit Transfer(gs_context_s* c) : ctx(c), lock(c->stage.mu) {}
     ~Transfer() { (void)hipStreamSynchronize(ctx->stream); }
-    // At least n words on the device.
+    // At least n words on the device, or NULL when there is no room for them
+    // (a call that starts with the state already changed, or reads results
+    // back from a full device, has to end without them).
     uint32_t* dev(size_t n) {
         Staging& s = ctx->stage;
         if (n > s.dev_words) {
             if (s.dev) dev_free(s.dev);
             s.dev = nullptr;
             s.dev_words = 0;
-            s.dev = (uint32_t*)dev_alloc(n * 4);
+            try {
+                s.dev = (uint32_t*)dev_alloc(n * 4);
+            } catch (const Error&) {
+                return nullptr;
+            }
             s.dev_words = n;
         }
         return s.dev;
@@ -214,7 +220,8 @@ static void trim(Staging& s) {
 // n words of each field from host arrays to consecutive slots.  Small groups
 // go as one block through pinned memory, which pays while the calls cost more
 // than the bytes (through the Python API, field by field / packed: 4,096
-// agents 298 / 101 us, 16,384 312 / 167 us, 65,536 397 / 416 us).
+// agents 298 / 101 us, 16,384 312 / 167 us, 65,536 397 / 416 us); the others,
+// and any without room for the staging, field by field.
 constexpr size_t kPackedUploadWords = kStageWords / 2;
 static void upload_words(gs_context_s* ctx, uint32_t n, const FieldWords& f, const uint32_t* const* host) {
     if (!n || !f.nf) return;
@@ -222,12 +229,12 @@ static void upload_words(gs_context_s* ctx, uint32_t n, const FieldWords& f, con
     const size_t words = (size_t)f.nf * n;
     Transfer t(ctx);
     uint32_t* hp = words <= kPackedUploadWords ? t.host(words) : nullptr;
-    if (!hp) {
+    uint32_t* dp = hp ? t.dev(words) : nullptr;
+    if (!dp) {
         for (int j = 0; j < f.nf; ++j) h2d(f.p[j], host[j], (size_t)n * 4, st);
         t.wait();
         return;
     }
-    uint32_t* dp = t.dev(words);
     for (int j = 0; j < f.nf; ++j) memcpy(hp + (size_t)j * n, host[j], (size_t)n * 4);
     h2d(dp, hp, words * 4, st);
     launch_unpack_fields(n, dp, f, st);
@@ -236,7 +243,8 @@ static void upload_words(gs_context_s* ctx, uint32_t n, const FieldWords& f, con
 
 // Each field's n slots to a host array in agent-index order (the host used to
 // wait for and permute every field: 4,096 agents 734 -> 91 us, 131,072 1,767 ->
-// 1,074 us, 1,048,576 21.7 -> 13.9 ms).
+// 1,074 us, 1,048,576 21.7 -> 13.9 ms; it still does where the device has no
+// room for the packed block).
 static void download_words(gs_context_s* ctx, uint32_t n, const uint32_t* ids, const FieldWords& f,
                            uint32_t* const* host) {
     if (!n || !f.nf) return;
@@ -245,6 +253,19 @@ static void download_words(gs_context_s* ctx, uint32_t n, const uint32_t* ids, c
     // Fields per pass: all, or as many as the staging holds (at least one).
     const int per = (int)std::min<size_t>(f.nf, std::max<size_t>(1, kStageWords / n));
     uint32_t* dp = t.dev((size_t)per * n + 1);
+    if (!dp) {
+        std::vector<uint32_t> id(n), v(n);
+        d2h(id.data(), ids, (size_t)n * 4, st);
+        t.wait();
+        for (uint32_t i : id)
+            if (i >= n) fail(GS_ERR_DEVICE, "agent id map corrupted");
+        for (int j = 0; j < f.nf; ++j) {
+            d2h(v.data(), f.p[j], (size_t)n * 4, st);
+            t.wait();
+            for (uint32_t s = 0; s < n; ++s) host[j][id[s]] = v[s];
+        }
+        return;
+    }
     uint32_t* hp = per == f.nf ? t.host((size_t)per * n + 1) : nullptr;
     uint32_t bad = 0;
     for (int j0 = 0; j0 < f.nf; j0 += per) {
@@ -785,8 +806,9 @@ static void begin_members(gs_group_s* g, uint32_t n) {
     g->idb[0].reserve(n);
     g->idb[1].reserve(n);
     g->slot_of_id.reserve(n);
-    // Here rather than at the first search, which may be recorded into a frame.
-    if (n <= kChunkMax) g->cbox.reserve(chunk_words(kChunkMax));
+    // Here rather than at the first search, which may be recorded into a frame,
+    // and for any n, so that a smaller upload later needs no memory.
+    g->cbox.reserve(chunk_words(kChunkMax));
     g->cbox_fresh = false;
     launch_iota(g->ids(), n, g->ctx->stream);
     g->n = n;
@@ -1173,6 +1195,23 @@ int gs_knn_download(gs_knn knn, uint32_t* idx, float* dist) {
         // staging holds (at least one).
         const size_t per = std::min(k, std::max<size_t>(1, kStageWords / (2 * n)));
         uint32_t* dp = t.dev(2 * per * n);
+        if (!dp) {
+            std::vector<uint32_t> ida(n), idb(B->n), vi(n);
+            std::vector<float> vd(n);
+            d2h(ida.data(), A->ids(), n * 4, st);
+            d2h(idb.data(), B->ids(), (size_t)B->n * 4, st);
+            for (size_t j = 0; j < k; ++j) {
+                d2h(vi.data(), knn->idx() + j * n, n * 4, st);
+                d2h(vd.data(), knn->dist() + j * n, n * 4, st);
+                t.wait();
+                for (size_t s = 0; s < n; ++s) {
+                    const size_t o = j * n + ida[s];
+                    if (idx) idx[o] = vi[s] < B->n ? idb[vi[s]] : UINT32_MAX;
+                    if (dist) dist[o] = vd[s];
+                }
+            }
+            return;
+        }
         uint32_t* hp = per == k ? t.host(2 * per * n) : nullptr;
         for (size_t j0 = 0; j0 < k; j0 += per) {
             const size_t rows = std::min(per, k - j0), words = rows * n;

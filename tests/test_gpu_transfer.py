@@ -64,3 +64,58 @@ def test_lists_in_agent_order(gs, ctx, orc, na, nb, k):
     np.testing.assert_array_equal(only, dist)
     for h in (knn, bins, A, B):
         h.close()
+
+
+def _same(a, b):
+    for f in AGENT_FIELDS + ("bits",):
+        np.testing.assert_array_equal(a[f], b[f], err_msg=f)
+
+
+# Without room on the device for the packed block the transfers go field by
+# field: an upload, which has changed its handle before, ends whole, and results
+# can be read back.
+def test_transfers_without_staging_memory(gs, orc):
+    c = gs.Context(0)  # no staging yet, and 50,000 agents take none
+    a, b = _state(50000), _state(5000)
+    A = gs.AgentGroup(c, a)
+    bins = gs.KNNBinData(c, (9, 9, 9), (50.0,) * 3, origin=(0.0,) * 3)
+    knn = gs.KNNData(c, 50000, 7)
+    gs.updateKNNDatabase(A, bins)  # storage order is cell order from here on
+    gs.findKNearestNeighbors(A, knn, bins, A, 1)
+    try:
+        capi.lib.gs_debug_fail_alloc_after(0)
+        _same(A.download(), a)
+        idx, dist = knn.download()
+        A.upload(b)
+        _same(A.download(), b)
+    finally:
+        capi.lib.gs_debug_fail_alloc_after(-1)
+    _same(A.download(), b)
+    q = np.unique(np.linspace(0, 49999, 200).astype(np.uint32))
+    r_idx, r_dist = orc.knn_brute(a.pos(), a.pos(), 7, True, queries=q)
+    np.testing.assert_array_equal(idx[:, q], r_idx[:, q])
+    np.testing.assert_array_equal(dist[:, q], r_dist[:, q])
+    for h in (knn, bins, A):
+        h.close()
+    c.close()
+
+
+def test_ensemble_transfers_without_staging_memory(gs):
+    c = gs.Context(0)
+    st, p = scenarios.boids_sphere(n=5000)
+    other, _ = scenarios.boids_sphere(n=5000, workload=2)
+    e = gs.Ensemble(c, [("boids", st, p)])
+    e.step(3)  # storage order is cell order from here on
+    try:
+        capi.lib.gs_debug_fail_alloc_after(0)
+        out = e.download(0)  # one word more than the upload's staging
+        e.upload(0, 0, other)
+        _same(e.download(0), other)
+    finally:
+        capi.lib.gs_debug_fail_alloc_after(-1)
+    _same(e.download(0), other)
+    e.upload(0, 0, st)
+    e.step(3)
+    _same(e.download(0), out)
+    e.close()
+    c.close()
