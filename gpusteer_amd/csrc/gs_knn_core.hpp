@@ -125,7 +125,8 @@ __device__ __forceinline__ float axis_gap(float q, int i0, int i1, float o, floa
 
 // Largest d2 from the query to the k neighbours of its previous exact result
 // (a valid upper bound on the current k-th distance: they are k distinct
-// candidates), or +inf when that result is incomplete.  The previous result
+// candidates), or +inf when that result is incomplete or one of them is now at
+// no distance (NaN).  The previous result
 // may be held at the previous storage order of A (row = its old slot) and of
 // B (val_map translates old B slots to current ones).  Unrolled over KMAX so
 // all loads of a level are in flight together.
@@ -148,10 +149,14 @@ __device__ __forceinline__ float seed_bound(const uint32_t* __restrict__ seed, u
     float4 p[KMAX];
 #pragma unroll
     for (int j = 0; j < KMAX; ++j) p[j] = bpos[v[j]];
-    float m = 0.f;
+    // The maximum of the bits: they order like the values, and a NaN lies above
+    // them all (fmaxf drops it).
+    uint32_t m = 0u;
 #pragma unroll
-    for (int j = 0; j < KMAX; ++j) m = fmaxf(m, sqdist4(qx, qy, qz, p[j]));
-    return m;
+    for (int j = 0; j < KMAX; ++j) m = max(m, __float_as_uint(sqdist4(qx, qy, qz, p[j])));
+    if (m <= 0x7F800000u) return __uint_as_float(m);
+    // A query that is no number itself has no candidates.
+    return qx == qx && qy == qy && qz == qz ? INFINITY : 0.f;
 }
 
 // Distance from the query to the nearest cell outside the box of ring R

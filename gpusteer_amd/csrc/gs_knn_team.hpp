@@ -253,7 +253,8 @@ template <int G, int KM, int RF> struct TeamList {
 };
 
 // Largest d2 to the k neighbours of the previous exact result (seed_bound's
-// value, the neighbours dealt to the team's lanes), +inf when incomplete.
+// value, the neighbours dealt to the team's lanes), +inf when incomplete or
+// when one is at no distance (NaN).
 template <int G, int KM, int RF>
 __device__ __forceinline__ float team_seed_bound(const TeamList<G, KM, RF>& L, bool active,
                                                  const uint32_t* __restrict__ seed, uint32_t nA, uint32_t row,
@@ -267,7 +268,9 @@ __device__ __forceinline__ float team_seed_bound(const TeamList<G, KM, RF>& L, b
             bad = true;
         } else {
             if (val_map) v = val_map[v];
-            m = fmaxf(m, sqdist4(qx, qy, qz, bpos[v]));
+            const float d2 = sqdist4(qx, qy, qz, bpos[v]);
+            m = fmaxf(m, d2);
+            bad = bad || (d2 != d2 && qx == qx && qy == qy && qz == qz);
         }
     }
     m = L.max_of(m);

@@ -100,3 +100,39 @@ def test_same_lists_as_one_lane(gs, ctx, n, cells, radius):
     for g, w in zip(got, want):
         np.testing.assert_array_equal(g[0], w[0])
         np.testing.assert_array_equal(g[1], w[1])
+
+
+# Exhaustive, local then chunks, teams, one lane per query, the split scan; the
+# group itself and another one.
+@pytest.mark.parametrize("na,nb,k,cells", [(100, 0, 7, (8, 8, 8)), (700, 100, 3, (8, 8, 8)), (700, 3000, 7, (12, 12, 12)),
+                                           (3000, 0, 7, (12, 12, 12)), (40000, 0, 16, (24, 24, 24)),
+                                           (131073, 0, 7, (36, 36, 36)), (131073, 0, 4, (36, 36, 36)),
+                                           (700, 3000, 20, (12, 12, 12))])
+def test_seed_with_lost_positions(gs, ctx, na, nb, k, cells):
+    """A neighbour of the previous result whose position is no number any more
+    bounds nothing: the list is that of a search without a seed."""
+    A, B = (_movers(gs, ctx, _points(n, n + k)) if n else None for n in (na, nb))
+    bins = gs.KNNBinData(ctx, cells, (SIZE,) * 3, origin=(0.0, 0.0, 0.0))
+    seeded, fresh = gs.KNNData(ctx, na, k), gs.KNNData(ctx, na, k)
+    groups = [A] + ([B] if B else [])
+    for step in range(2):
+        for G in groups:
+            if step:
+                gs.updateGroup(G, 0.01, capi.GS_MODE_GPUREF)
+            gs.updateKNNDatabase(G, bins)
+        gs.findKNearestNeighbors(A, seeded, bins, B or A, 1)
+    gs.findKNearestNeighbors(A, fresh, bins, B or A, 1, capi.GS_KNN_NO_SEED)
+    assert np.isnan((B or A).download().pos()).any()
+    got, want = seeded.download(), fresh.download()
+    np.testing.assert_array_equal(got[0], want[0])
+    np.testing.assert_array_equal(got[1], want[1])
+    for h in [seeded, fresh, bins] + groups:
+        h.close()
+
+
+def _movers(gs, ctx, pos):
+    """A group of which every 29th agent loses its position at the first update."""
+    n = pos.shape[0]
+    st = scenarios.make_agents(pos, np.tile([[0.0, 0.0, 1.0]], (n, 1)), np.ones(n), 0.5, 1.0, 1.0)
+    st.arrays["speed"][::29] = np.nan
+    return gs.AgentGroup(ctx, st)
