@@ -12,7 +12,9 @@
 // each other's state: group 0's separation from group 1 reads group 1's
 // positions before group 1's walls move them, which are the snapshot's, and
 // everything else reads the positions that the walls have left, which the
-// second phase only reads (new positions go to the alternate buffers).
+// second phase only reads.  Both phases write positions and forward vectors to
+// the alternate buffers: a frame then leaves every field in the buffer in which
+// the separate calls would, which recorded frames are compared by.
 #include "gs_knn_chunks.hpp"
 #include "gs_ops.hpp"
 
@@ -103,7 +105,7 @@ struct PairAgents {
     Agents A;
     const uint32_t *kown, *kother, *kwalls, *kobs;
     uint32_t k[4];
-    float *npx, *npy, *npz, *nfx, *nfy, *nfz;  // alternate buffers
+    float *npx, *npy, *npz, *nfx, *nfy, *nfz;  // A's alternate buffers
     float goal[3];
 };
 struct PairSteer {
@@ -132,8 +134,8 @@ __global__ __launch_bounds__(kBlock) void k_pair_avoid(PairSteer P) {
                     bits);
     avoid_obstacles_one(pos, dir, side, ld3(A.ux, A.uy, A.uz, i), radius, speed, G.kobs + i, G.n, G.k[3], P.nO, P.ox, P.oy,
                         P.oz, P.orad, P.mt_obs, P.w_obs, steering, bits);
-    st3(A.px, A.py, A.pz, i, pos);
-    st3(A.fx, A.fy, A.fz, i, dir);
+    st3(G.npx, G.npy, G.npz, i, pos);
+    st3(G.nfx, G.nfy, G.nfz, i, dir);
     st3(A.gx, A.gy, A.gz, i, steering);
     A.bits[i] = bits;
 }
@@ -187,16 +189,26 @@ void launch_pair_steer(gs_group_s* const g[2], gs_group_s* W, gs_group_s* O, gs_
         PairAgents& a = P.a[i];
         a.n = g[i]->n;
         n = std::max(n, a.n);
-        a.A = g[i]->dev_agents();
         a.kown = knn[4 * i]->idx();
         a.kother = knn[4 * i + 1]->idx();
         a.kwalls = knn[4 * i + 2]->idx();
         a.kobs = knn[4 * i + 3]->idx();
         for (int j = 0; j < 4; ++j) a.k[j] = knn[4 * i + j]->k;
-        float** out[6] = {&a.npx, &a.npy, &a.npz, &a.nfx, &a.nfy, &a.nfz};
-        for (int j = 0; j < 6; ++j) *out[j] = g[i]->Falt(j);
         for (int j = 0; j < 3; ++j) a.goal[j] = s->goal[i][j];
     }
+    // Where the next kernel reads and writes positions and forward vectors.
+    auto state = [&] {
+        for (int i = 0; i < 2; ++i) {
+            PairAgents& a = P.a[i];
+            a.A = g[i]->dev_agents();
+            float** out[6] = {&a.npx, &a.npy, &a.npz, &a.nfx, &a.nfy, &a.nfz};
+            for (int j = 0; j < 6; ++j) *out[j] = g[i]->Falt(j);
+        }
+    };
+    auto written = [&] {
+        for (int i = 0; i < 2; ++i)
+            for (int j = 0; j < 6; ++j) g[i]->flip(j);
+    };
     P.spos1 = g[1]->spos.p;
     P.nW = W->n;
     P.nO = O->n;
@@ -219,13 +231,16 @@ void launch_pair_steer(gs_group_s* const g[2], gs_group_s* W, gs_group_s* O, gs_
     hipStream_t st = g[0]->ctx->stream;
     const unsigned block = agent_block(n);
     const dim3 grid(agent_blocks(n), 2);
+    state();
     k_pair_avoid<<<grid, block, 0, st>>>(P);
     GS_LAUNCHED("k_pair_avoid");
+    written();
+    state();
     if (s->mode == GS_MODE_GPUREF) k_pair_finish<GS_MODE_GPUREF><<<grid, block, 0, st>>>(P);
     else k_pair_finish<GS_MODE_OPENSTEER><<<grid, block, 0, st>>>(P);
     GS_LAUNCHED("k_pair_finish");
+    written();
     for (int i = 0; i < 2; ++i) {
-        for (int j = 0; j < 6; ++j) g[i]->flip(j);
         g[i]->mark_written(kFSteer | 0x3Fu, true);
         g[i]->mark_integrated();
     }

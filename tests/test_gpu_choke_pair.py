@@ -84,3 +84,33 @@ def test_equals_separate_calls(gs, ctx, n0, n1, k, mode, cells, obstacles, walls
     _equal(_result(G2, knns2, bins2.num_cells), want)
     for h in [bins, W, O, bins2, W2, O2] + G + G2 + [x for ks in knns + knns2 for x in ks]:
         h.close()
+
+
+def test_buffers_end_as_with_separate_calls(gs, ctx):
+    """A recorded frame can be replayed when it ends in the buffers in which it
+    began: searches for display before the frame's own make it so, with the
+    separate calls and with the joint frame."""
+    sc = _scenario(900, 700, 9.0, 0, (40, 1, 40))
+    results = []
+    for calls in (choke_step_calls, step_choke):
+        bins, G, W, O, knns = _world(gs, ctx, sc, 7)
+
+        def frame():
+            for g in G:
+                gs.updateKNNDatabase(g, bins)
+            for g, other, (own, oth, wall, obs) in zip(G, G[::-1], knns):
+                gs.findKNearestNeighbors(g, own, bins, g, 1)
+                gs.findKNearestNeighborsWithin(g, oth, bins, other, sc.other_radius, 1)
+                gs.findKNearestNeighbors(g, wall, bins, W, 1)
+                gs.findKNearestNeighbors(g, obs, bins, O, 1)
+            calls(G, knns, W, O, bins, sc)
+
+        for _ in range(2):
+            frame()
+        with ctx.record(frame) as f:
+            f.launch(1)
+            f.launch(5)
+        results.append(_result(G, knns, bins.num_cells))
+        for h in [bins, W, O] + G + [x for ks in knns for x in ks]:
+            h.close()
+    _equal(*results)
