@@ -220,25 +220,24 @@ static void trim(Staging& s) {
 // n words of each field from host arrays to consecutive slots.  Small groups
 // go as one block through pinned memory, which pays while the calls cost more
 // than the bytes (through the Python API, field by field / packed: 4,096
-// agents 298 / 101 us, 16,384 312 / 167 us, 65,536 397 / 416 us); the others,
-// and any without room for the staging, field by field.
+// agents 298 / 99 us, 16,384 312 / 129 us, 65,536 385 / 416 us); the others,
+// and any without room for the staging, field by field.  Queued only: the
+// caller looks at the host arrays while they copy, then waits (waiting first:
+// 65,536 agents 385 -> 536 us, 131,072 600 -> 800 us).
 constexpr size_t kPackedUploadWords = kStageWords / 2;
-static void upload_words(gs_context_s* ctx, uint32_t n, const FieldWords& f, const uint32_t* const* host) {
+static void upload_words(Transfer& t, uint32_t n, const FieldWords& f, const uint32_t* const* host) {
     if (!n || !f.nf) return;
-    hipStream_t st = ctx->stream;
+    hipStream_t st = t.ctx->stream;
     const size_t words = (size_t)f.nf * n;
-    Transfer t(ctx);
     uint32_t* hp = words <= kPackedUploadWords ? t.host(words) : nullptr;
     uint32_t* dp = hp ? t.dev(words) : nullptr;
     if (!dp) {
         for (int j = 0; j < f.nf; ++j) h2d(f.p[j], host[j], (size_t)n * 4, st);
-        t.wait();
         return;
     }
     for (int j = 0; j < f.nf; ++j) memcpy(hp + (size_t)j * n, host[j], (size_t)n * 4);
     h2d(dp, hp, words * 4, st);
     launch_unpack_fields(n, dp, f, st);
-    t.wait();
 }
 
 // Each field's n slots to a host array in agent-index order (the host used to
@@ -843,7 +842,8 @@ int gs_group_upload_agents(gs_group g, uint32_t n, const gs_agents* host) {
         }
         f.p[kFields] = g->bits();
         src[kFields] = n ? host->bits : nullptr;
-        upload_words(g->ctx, n, f, src);
+        Transfer t(g->ctx);
+        upload_words(t, n, f, src);
         // Fields with one bit pattern in every slot (positions excluded).
         if (n) {
             for (int j = 3; j < kFields; ++j) {
@@ -859,7 +859,7 @@ int gs_group_upload_agents(gs_group g, uint32_t n, const gs_agents* host) {
             for (uint32_t i = 0; i < n && zero; ++i) zero = host->bits[i] == 0u;
             g->bits_zero = zero;
         }
-        GS_HIP(hipStreamSynchronize(g->ctx->stream));
+        t.wait();
     });
 }
 
@@ -2041,8 +2041,9 @@ int gs_ensemble_upload_agents(gs_ensemble e, uint32_t scenario, uint32_t group, 
         f.p[kFields] = e->bits() + P.a0;
         src[kFields] = bits.data();
         launch_iota(e->ids() + P.a0, P.n, st);
-        upload_words(e->ctx, P.n, f, src);
-        GS_HIP(hipStreamSynchronize(st));
+        Transfer t(e->ctx);
+        upload_words(t, P.n, f, src);
+        t.wait();
         e->seeded = false;
         // Which of the never-written fields hold one value in this population
         // (bit patterns), and so need not move in the counting sort.
