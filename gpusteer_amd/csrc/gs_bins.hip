@@ -209,6 +209,18 @@ __global__ __launch_bounds__(kBlock) void k_scan_add(uint32_t C, const uint32_t*
 constexpr int kScanOneThreads = 1024;
 constexpr uint32_t kScanOneCells = 16 * kScanOneThreads;
 constexpr uint32_t kScanOneAgents = 16 * kScanOneThreads;
+// Where one block pays.  The scan alone replaces two launches by one whose time
+// grows with the lattice; the scatter in it replaces a third one and adds 0.75
+// us per 1,024 agents.  Whole build, us, passes in launches of their own / in
+// one block: 500 agents on 12,167 cells 15.2 / 13.5, on 15,625 15.3 / 15.4;
+// 4,096 on 4,096 cells 15.8 / 13.1, on 12,167 15.8 / 15.6; 6,000 on 1,728 15.2 /
+// 15.3, on 8,000 16.0 / 16.1; 8,192 on 4,096 16.0 / 16.2, 16,384 on 4,096 19.3 /
+// 23.0 (with the scan alone 17).
+constexpr uint32_t kScanAloneCells = 12 * kScanOneThreads;
+constexpr uint32_t kScatterOneAgents = 5 * kScanOneThreads, kScatterOneSum = 10 * kScanOneThreads;
+static bool scatter_in_scan(uint32_t n, uint32_t C) {
+    return n > 0 && n <= kScatterOneAgents && C <= kScanOneCells && n + C / 2 <= kScatterOneSum;
+}
 __device__ __forceinline__ void scan_one(uint32_t C, uint32_t* __restrict__ count, uint32_t* start, uint32_t n,
                                          const uint32_t* __restrict__ key, const uint32_t* __restrict__ rank,
                                          const uint32_t* __restrict__ ids, uint32_t* __restrict__ id_tmp) {
@@ -454,7 +466,7 @@ __global__ __launch_bounds__(kBlock) void k_reorder_free(uint32_t n, uint32_t C,
 }
 
 void launch_scan_counts(uint32_t* count, uint32_t* start, uint32_t C, hipStream_t st) {
-    if (C <= kScanOneCells) {
+    if (C <= kScanAloneCells) {
         k_scan_one<<<1, kScanOneThreads, 0, st>>>(C, count, start, 0, nullptr, nullptr, nullptr, nullptr);
         GS_LAUNCHED("k_scan_one");
         return;
@@ -603,7 +615,7 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
     free_order = free_order && lazy && n > 0;
     // With k_reorder_free the offsets within the tiles use the scatter's
     // buffer.
-    const bool free_tiles = free_order && C > kScanOneCells && C <= n && ntiles <= kScanFusedTiles;
+    const bool free_tiles = free_order && C > kScanAloneCells && C <= n && ntiles <= kScanFusedTiles;
     float wcv[3] = {0, 0, 0}, wsv[3] = {0, 0, 0};
     if (wc) memcpy(wcv, wc, sizeof wcv);
     if (ws) memcpy(wsv, ws, sizeof wsv);
@@ -614,7 +626,7 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
         GS_LAUNCHED("k_bin_key");
     }
     // Small groups on small lattices: scan and scatter in one launch.
-    const bool one = n > 0 && n <= kScanOneAgents && C <= kScanOneCells && !free_order;
+    const bool one = !free_order && scatter_in_scan(n, C);
     if (one) {
         k_scan_one<<<1, kScanOneThreads, 0, st>>>(C, g->count.p, g->start.p, n, g->key.p, g->rank.p, g->ids(),
                                                   g->id_tmp.p);

@@ -13,7 +13,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n,cells", [
     (1, (1, 1, 1)), (2000, (32, 32, 16)), (2000, (32, 32, 17)), (16384, (16, 16, 16)), (16385, (16, 16, 16)),
-    (16384, (16385, 1, 1)), (16385, (128, 128, 1)), (50000, (1, 16383, 1)), (9000, (3, 2, 1))])
+    (16384, (16385, 1, 1)), (16385, (128, 128, 1)), (50000, (1, 16383, 1)), (9000, (3, 2, 1)),
+    (5120, (10240, 1, 1)), (5120, (1, 10242, 1)), (5121, (4, 4, 4)), (4096, (12288, 1, 1)), (4096, (1, 1, 12289)),
+    (2048, (16384, 1, 1)), (2049, (16384, 1, 1))])
 def test_build_is_the_stable_sort(gs, ctx, orc, n, cells):
     print(f"case n={n} cells={cells}", flush=True)
     g = np.random.default_rng(n)
@@ -41,7 +43,7 @@ def test_build_is_the_stable_sort(gs, ctx, orc, n, cells):
 
 @pytest.mark.parametrize("n,cells,wrap,mode", [
     (3000, (12, 12, 12), 1, 0), (20000, (16, 16, 16), 0, 1), (20001, (26, 26, 26), 0, 0), (40000, (32, 32, 32), 1, 0),
-    (40000, (36, 36, 36), 1, 1), (70000, (32, 32, 64), 0, 0)])
+    (40000, (36, 36, 36), 1, 1), (70000, (32, 32, 64), 0, 0), (20000, (24, 24, 24), 1, 0), (20000, (1, 96, 128), 0, 0)])
 def test_one_call_of_many_steps_equals_many_calls(gs, ctx, n, cells, wrap, mode):
     """The whole state, the storage order, the bins and the lists."""
     st, p = scenarios.boids_sphere(n=n)
