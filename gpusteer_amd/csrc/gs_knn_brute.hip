@@ -35,7 +35,10 @@
 // on 1,024 SIMDs, 27 us; measured 103 us, the rest being the minima and
 // compares of the products (four per instruction and lane) and the staging,
 // which four wavefronts per SIMD overlap only in part.  One lane per query with
-// a serial insertion per pair took 2,148 us (64 blocks on 256 CUs).
+// a serial insertion per pair takes 2,148 us (64 blocks on 256 CUs); few points
+// for many queries are still searched that way (brute_by_lanes).
+#include <algorithm>
+
 #include "gs_knn_core.hpp"
 
 namespace gs {
@@ -274,13 +277,15 @@ __global__ __launch_bounds__(kBruteThreads) void k_knn_brute(
         float lim = lds_lim[ql];
         int cnt = 0;
         // Adds each lane's point (when it has one) with d2 <= lim.
+        uint64_t worst = ~0ull;  // the k-th key once k are known: most ties lie beyond it
         auto add = [&](bool has, uint32_t b, float x, float y, float z, uint32_t id) {
             const float d2 = sqdist(qx, qy, qz, x, y, z);
-            const bool pass = has && d2 <= lim;
+            const uint64_t mk = make_key(d2, id);
+            const bool pass = has && d2 <= lim && mk <= worst;
             const uint64_t v = __ballot(pass);
             if (pass) {
                 const int at = cnt + __popcll(v & ((1ull << lane) - 1ull));
-                key[at] = make_key(d2, id);
+                key[at] = mk;
                 slot[at] = b;
             }
             cnt += __popcll(v);
@@ -298,7 +303,7 @@ __global__ __launch_bounds__(kBruteThreads) void k_knn_brute(
                 add(b0 + lane < nB && !(self && b == q), b, bx[b], by[b], bz[b], bids[b]);
                 if (cnt + 64 > kBruteCap) {
                     cnt = brute_reduce(key, slot, cnt, k);
-                    if (cnt == (int)k) lim = fminf(lim, __uint_as_float((uint32_t)(key[k - 1u] >> 32)));
+                    if (cnt == (int)k) worst = key[k - 1u];
                 }
             }
         }
@@ -313,11 +318,79 @@ __global__ __launch_bounds__(kBruteThreads) void k_knn_brute(
     }
 }
 
+// One lane per query, B staged through LDS in tiles of one block (positions and
+// agent indices).  Bound by the serial insertions of a lane, about 0.2 (k = 1)
+// to 0.6 us (k = 32) per point while the chip is not full.
+template <int KMAX>
+__global__ __launch_bounds__(kBlock) void k_knn_brute_lanes(
+    uint32_t nA, const float* __restrict__ ax, const float* __restrict__ ay, const float* __restrict__ az, uint32_t nB,
+    const float* __restrict__ bx, const float* __restrict__ by, const float* __restrict__ bz,
+    const uint32_t* __restrict__ bids, int self, uint32_t k, float cap2, uint32_t* __restrict__ out_idx,
+    float* __restrict__ out_dist) {
+    __shared__ float tx[kBlock], ty[kBlock], tz[kBlock];
+    __shared__ uint32_t tid[kBlock];
+    const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool active = q < nA;
+    const float qx = active ? ax[q] : 0.f, qy = active ? ay[q] : 0.f, qz = active ? az[q] : 0.f;
+    TopK<KMAX> h;
+    h.init(k);
+    for (uint32_t base = 0; base < nB; base += kBlock) {
+        const uint32_t t = base + threadIdx.x;
+        if (t < nB) {
+            tx[threadIdx.x] = bx[t];
+            ty[threadIdx.x] = by[t];
+            tz[threadIdx.x] = bz[t];
+            tid[threadIdx.x] = bids[t];
+        }
+        __syncthreads();
+        const uint32_t m = min((uint32_t)kBlock, nB - base);
+        if (active) {
+            for (uint32_t j = 0; j < m; ++j) {
+                const uint32_t b = base + j;
+                if (self && b == q) continue;
+                const float d2 = sqdist(qx, qy, qz, tx[j], ty[j], tz[j]);
+                const uint64_t kk = make_key(d2, tid[j]);
+                if (d2 <= cap2 && h.accepts(kk)) h.push(kk, b);
+            }
+        }
+        __syncthreads();
+    }
+    if (active) h.store(k, nA, q, out_idx, out_dist);
+}
+
+// Whether few points meet many queries, where a lane per query is faster: the
+// matrix form spends about 1.6 us per 1,000 queries beyond 4,096 on its blocks'
+// set-up and selection whatever nB, the lanes a time per point that grows with
+// the list and, once the chip is full, with the queries (short lists fill it
+// later).  Lanes / matrix, us, k = 7: 4,096 queries 7 / 10 at 16 points, 16 / 12
+// at 50; 16,384 29 / 33 at 100, 52 / 32 at 200; 65,536 99 / 117 at 400, 178 / 120
+// at 800; 131,072 38 / 235 at 100, 222 / 236 at 800; 500,000 940 / 1,038 at
+// 1,600.  k = 16: 16,384 42 / 48 at 100, 78 / 60 at 200; 131,072 227 / 255 at 400,
+// 422 / 256 at 800.  k = 32: 16,384 36 / 39 at 50, 65 / 48 at 100; 131,072 441 /
+// 537 at 400, 880 / 294 at 800.
+static bool brute_by_lanes(uint32_t nA, uint32_t nB, uint32_t k) {
+    const double point = k <= 8 ? 18.0 : (k <= 16 ? 24.0 : 30.0);
+    const double full = std::max(1.0, nA / 98304.0 * std::min(k + 2u, 12u) / 12.0);
+    return nB * point * full <= 336.0 + (std::max(nA, 4096u) - 4096u) / 7.5;
+}
+
 void launch_knn_brute(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2) {
     const uint32_t nA = A->n;
     if (nA == 0) return;
     hipStream_t st = A->ctx->stream;
     const int self = A == B ? 1 : 0;
+    if (brute_by_lanes(nA, B->n, out->k)) {
+#define GS_BRUTE_LANES(KM)                                                                                           \
+    k_knn_brute_lanes<KM><<<blocks_for(nA), kBlock, 0, st>>>(nA, A->F(0), A->F(1), A->F(2), B->n, B->F(0), B->F(1), \
+                                                             B->F(2), B->ids(), self, out->k, cap2, out->idx_alt(), \
+                                                             out->dist_alt())
+        if (out->k <= 8) GS_BRUTE_LANES(8);
+        else if (out->k <= 16) GS_BRUTE_LANES(16);
+        else GS_BRUTE_LANES(32);
+#undef GS_BRUTE_LANES
+        GS_LAUNCHED("k_knn_brute_lanes");
+        return;
+    }
 #define GS_BRUTE(T)                                                                                                 \
     k_knn_brute<T><<<blocks_for(nA, 16 * T), kBruteThreads, 0, st>>>(nA, A->F(0), A->F(1), A->F(2), B->n, B->F(0),   \
                                                                      B->F(1), B->F(2), B->ids(), self, out->k, cap2, \

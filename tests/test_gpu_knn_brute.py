@@ -67,6 +67,22 @@ def test_tile_edges(gs, ctx, na, nb, k):
     bins.close()
 
 
+# Both sides of the line between a lane per query and the matrix cores.
+@pytest.mark.parametrize("na,nb,k", [
+    (100, 18, 7), (100, 19, 7), (17, 0, 7), (16384, 109, 7), (16384, 110, 7), (20000, 100, 16), (20000, 80, 32),
+    (131072, 958, 7), (131072, 960, 7), (300001, 700, 5), (100000, 1, 16), (4097, 0, 1)])
+def test_few_points_for_many_queries(gs, ctx, na, nb, k):
+    print(f"case na={na} nb={nb} k={k}", flush=True)
+    g = np.random.default_rng(na + nb)
+    a = g.uniform(-50, 50, (na, 3)).astype(np.float32)
+    b = g.uniform(-50, 50, (nb, 3)).astype(np.float32) if nb else None
+    if nb > 20:
+        b[:9], b[11] = b[9], (np.nan, 0.0, np.inf)
+    bins = gs.KNNBinData(ctx, (7, 7, 7), (100.0,) * 3)
+    _check(gs, ctx, a, b, k, bins)
+    bins.close()
+
+
 def _cases():
     g = np.random.default_rng(1)
     u = g.uniform(-1, 1, (2500, 3))
