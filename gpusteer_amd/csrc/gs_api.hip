@@ -1287,12 +1287,25 @@ static bool prefer_exhaustive(const gs_group_s* B, const GridDev& g, uint32_t ce
     return reach_cells(g, cells, max_distance) * 4 >= B->n;
 }
 
-// A small query group searching another small group over a wide reach: the
-// split exhaustive scan fills the chip where a one-lane-per-query search
-// would run as a few dozen wavefronts, each walking the cells around a query
-// that the other group may be far from.  A group's search of itself (its
-// points are where its queries are) and a narrowly capped search stay in the
-// bins.
+// Points of B that a capped search would reach if they lay evenly over the
+// lattice.
+static uint64_t points_in_reach(const gs_group_s* B, const GridDev& g, uint32_t cells, float max_distance) {
+    return reach_cells(g, cells, max_distance) * B->n / cells;
+}
+// A search without a seed looks for a bound first when it reaches more points
+// than this: with fewer the bound costs more than it saves (131,072 queries of
+// 1,254 walls, k = 7, bound first / not: 14 in reach 49 / 28 us, 102 in reach 53 /
+// 71, all 54 / 332).
+constexpr uint64_t kWideCapPoints = 64;
+
+// A small query group searching another small group over a wide reach: one lane
+// per query would run as a few dozen wavefronts, each walking the cells around
+// a query that the other group may be far from.  Such searches take the cells
+// around the query and then B's chunks by teams of lanes (launch_knn_chunks),
+// lists too long for those the split exhaustive scan; the range count says
+// that there are points enough for either to share out.  A group's search of
+// itself (its points are where its queries are) and a narrowly capped search
+// stay in the bins.
 static bool prefer_split(const gs_group_s* A, const gs_group_s* B, const GridDev& g, uint32_t cells,
                          float max_distance) {
     return A != B && A->n <= kSplitMaxA && B->n <= kSplitMaxB && (uint64_t)A->n * B->n <= kSplitMaxPairs &&
@@ -1319,16 +1332,18 @@ static void find_knn(gs_group A, gs_knn out, gs_bins bins, gs_group B, uint32_t 
     const bool split = !(flags & GS_KNN_BINNED) && prefer_split(A, B, bins->g, bins->cells, max_distance);
     const bool exhaustive =
         !split && !(flags & GS_KNN_BINNED) && prefer_exhaustive(B, bins->g, bins->cells, max_distance);
-    if ((split || exhaustive) && out->k <= kChunkMaxK && B->n <= kChunkMax) {
-        const Seed sd = seed_for(out, A, B, flags);
-        launch_knn_chunks(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map, split ? std::max(search_radius, 1u) : 0u);
-    } else if (split) {
-        const Seed sd = seed_for(out, A, B, flags);
-        launch_knn_split(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map);
-    } else if (exhaustive) {
+    const Seed sd = seed_for(out, A, B, flags);
+    const uint64_t reach = points_in_reach(B, bins->g, bins->cells, max_distance);
+    if (exhaustive && out->k > kChunkMaxK) {
         launch_knn_snap_brute(A, out, B, cap2);
+    } else if ((split || exhaustive) && out->k <= kChunkMaxK && B->n <= kChunkMax) {
+        // The cells around a query hold nothing of a sparse B.
+        const bool local = split && !prefer_exhaustive(B, bins->g, bins->cells, max_distance);
+        launch_knn_chunks(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map, local ? std::max(search_radius, 1u) : 0u,
+                          reach > kWideCapPoints);
+    } else if (split) {
+        launch_knn_split(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map);
     } else {
-        const Seed sd = seed_for(out, A, B, flags);
         launch_knn_binned(A, out, B, search_radius, cap2, sd.seed, sd.row_map, sd.val_map);
     }
     out->cur ^= 1;

@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kBlock) void e_knn_team(
             thr = team_seed_bound(L, active, out.seed_self, N, active ? new_to_old[s] : 0u, N, old_to_new, q.x, q.y,
                                   q.z, spos);
         const FlatQuery Q{q.x, q.y, q.z, thr, s, active};
-        knn_search_team(L, Q, P.g, N, spos, start + P.c0);
+        knn_search_team<false>(L, Q, P.g, N, spos, start + P.c0, thr == INFINITY);
         store(out.self, true);
         return;
     }
@@ -262,9 +262,10 @@ __global__ __launch_bounds__(kBlock) void e_knn_team(
         if (out.seed_other)
             thr = fminf(cap2, team_seed_bound(L, active, out.seed_other, N, active ? new_to_old[s] : 0u, N, old_to_new,
                                               q.x, q.y, q.z, spos));
+        const bool bound_first = thr == INFINITY;
         if (active && box_beyond(out.box + 6 * (size_t)P.other, q.x, q.y, q.z, cap2)) thr = -1.f;
         const FlatQuery Q{q.x, q.y, q.z, thr, UINT32_MAX, active};
-        knn_search_team(L, Q, O.g, N, spos, start + O.c0);
+        knn_search_team<false>(L, Q, O.g, N, spos, start + O.c0, bound_first);
     }
     store(out.other, true);
     const EnsScen& S = E.scens[P.scen];

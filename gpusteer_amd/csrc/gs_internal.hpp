@@ -535,7 +535,7 @@ constexpr size_t chunk_words(uint32_t n) { return 6 * (((size_t)n + 63) / 64); }
 // local: 0, or the cell radius of the box around the query that is searched
 // first (of B's lattice; at most kSplitMaxA queries).
 void launch_knn_chunks(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, const uint32_t* seed,
-                       const uint32_t* row_map, const uint32_t* val_map, uint32_t local);
+                       const uint32_t* row_map, const uint32_t* val_map, uint32_t local, bool wide_cap);
 // The chunk boxes of B's snapshot, if they are not the current one's.
 void launch_chunk_boxes(gs_group_s* B);
 // Whether this thread records a frame (its kernels run at the replays, so

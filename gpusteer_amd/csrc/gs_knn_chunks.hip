@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kBlock) void k_knn_chunks(uint32_t nA, const float4
                                                        const float* __restrict__ boxes,
                                                        const uint32_t* __restrict__ bstart, GridDev g,
                                                        const uint32_t* __restrict__ box, int self, uint32_t k,
-                                                       float cap2, const uint32_t* __restrict__ seed,
+                                                       float cap2, int wide_cap, const uint32_t* __restrict__ seed,
                                                        const uint32_t* __restrict__ row_map,
                                                        const uint32_t* __restrict__ val_map,
                                                        uint32_t* __restrict__ out_idx, float* __restrict__ out_dist) {
@@ -63,15 +63,17 @@ __global__ __launch_bounds__(kBlock) void k_knn_chunks(uint32_t nA, const float4
         if (seed)
             thr = fminf(cap2, team_seed_bound(L, active, seed, nA, (active && row_map) ? row_map[s] : s, nB, val_map, q.x,
                                               q.y, q.z, bpos));
+        // A list that the cap left short last time needs no other bound.
+        const bool bound_first = (!seed && wide_cap) || thr == INFINITY;
         // As k_knn_binned: no candidate within the cap of B's bounding box.
         if (box && active && box_beyond(box, q.x, q.y, q.z, cap2)) thr = -1.f;
         FlatQuery Q{q.x, q.y, q.z, thr, self ? s : UINT32_MAX, active};
         bool found = false;
         if (Local) {
-            found = knn_search_team(L, Q, g, nB, bpos, bstart, (int)((nB + 63u) / 64u));
+            found = knn_search_team<true>(L, Q, g, nB, bpos, bstart, bound_first, (int)((nB + 63u) / 64u));
             Q.thr = L.lim;
         }
-        if (!found) knn_chunks_team(L, Q, Q.thr == (Local ? cap2 : INFINITY), nB, bpos, boxes);
+        if (!found) knn_chunks_team(L, Q, bound_first, nB, bpos, boxes);
     }
     if (active) L.store(nA, s, out_idx, out_dist);
 }
@@ -81,14 +83,23 @@ __global__ __launch_bounds__(kBlock) void k_knn_chunks(uint32_t nA, const float4
 // no seed, before).  Two groups of 5,000 (k = 7, cap of ten cells, 100 x 1 x
 // 100 cells): 47 us by ranges per block and a merge, 50 over the chunks alone (a
 // chunk is a strip across the lattice, and one query without a seed under a
-// wide cap holds its block up), 16 + 3 with the cells around the
-// query first and rings without an end, 20 + 3 here.  The end is at as many
-// columns as chunks: with 5,000 queries of 5,000 points (k = 7, 32^3 cells)
-// mixed / apart / about one cluster, seeded, cap of ten cells: chunks alone 15
-// / 5 / 15 us, no end 20 / 59 / 125, here 27 / 11 / 24; unseeded 71 / 4 / 205,
-// 28 / 58 / 230 and 51 / 11 / 84.
+// wide cap holds its block up), 16 + 3 with the cells around the query first
+// and rings without an end, 13 + 3 here.  The rings end at as many columns as
+// chunks, at more cells than points, and at a ring full of points: with 5,000
+// queries of 5,000 points (k = 7, 32^3 cells) mixed / apart / about one cluster,
+// seeded: chunks alone 15 / 5 / 15 us, no end 20 / 59 / 125, here 17 / 14 / 15;
+// unseeded, no cap 71 / 4 / 205, 28 / 58 / 230, here 26 / 25 / 36 (100 x 1 x 100
+// cells 16 / 41 / 69; by ranges and a merge 100 / 117 / 98).
+//
+// A whole wavefront per query where there are few queries and many points; wider
+// lattices than one cell high have more columns to share.  16 / 64 lanes, us, k
+// = 7, seeded: 500 queries of 16,000 points mixed 14 / 11, apart 26 / 14, about
+// one cluster 65 / 16; 2,048 of 16,384 14 / 12, 27 / 15, 69 / 19; 5,000 of 5,000
+// 28 / 17, 17 / 15, 26 / 15, but 13 / 15, 20 / 23, 27 / 23 on 100 x 1 x 100 cells;
+// 16,384 of 4,096 33 / 39, 19 / 31, 28 / 31 and 15 / 36, 25 / 49, 30 / 50.
+constexpr uint32_t kTeam64Max = 4096, kTeam64MaxColumns = 8192, kTeam64MinPoints = 257;
 void launch_knn_chunks(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, const uint32_t* seed,
-                       const uint32_t* row_map, const uint32_t* val_map, uint32_t local) {
+                       const uint32_t* row_map, const uint32_t* val_map, uint32_t local, bool wide_cap) {
     const uint32_t nA = A->n;
     if (nA == 0) return;
     launch_chunk_boxes(B);
@@ -97,9 +108,17 @@ void launch_knn_chunks(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, 
 #define GS_CHUNKS(G, KM, RF, Local)                                                                            \
     k_knn_chunks<G, KM, RF, Local><<<blocks_for(nA, team_queries<G>()), kBlock, 0, A->ctx->stream>>>(          \
         nA, A->spos.p, B->n, B->spos.p, B->cbox.p, B->start.p, B->bin_grid, box, A == B ? 1 : 0, out->k, cap2, \
-        seed, row_map, val_map, out->idx_alt(), out->dist_alt())
+        wide_cap ? 1 : 0, seed, row_map, val_map, out->idx_alt(), out->dist_alt())
     static_assert(kSplitMaxA <= kTeam16Max, "a local search has 16 lanes per query");
-    if (local >= 2 && out->k <= 8) GS_CHUNKS(16, 8, 2, true);
+    const bool columns = local && B->bin_grid.dx > 1 && B->bin_grid.dy > 1;
+    if (nA <= (columns ? kTeam64MaxColumns : kTeam64Max) && B->n >= kTeam64MinPoints) {
+        if (local >= 2 && out->k <= 8) GS_CHUNKS(64, 8, 2, true);
+        else if (local >= 2) GS_CHUNKS(64, 16, 2, true);
+        else if (local && out->k <= 8) GS_CHUNKS(64, 8, 1, true);
+        else if (local) GS_CHUNKS(64, 16, 1, true);
+        else if (out->k <= 8) GS_CHUNKS(64, 8, 1, false);
+        else GS_CHUNKS(64, 16, 1, false);
+    } else if (local >= 2 && out->k <= 8) GS_CHUNKS(16, 8, 2, true);
     else if (local >= 2) GS_CHUNKS(16, 16, 2, true);
     else if (local && out->k <= 8) GS_CHUNKS(16, 8, 1, true);
     else if (local) GS_CHUNKS(16, 16, 1, true);

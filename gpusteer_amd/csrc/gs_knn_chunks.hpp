@@ -22,11 +22,13 @@ __device__ __forceinline__ float chunk_gap2(const float* __restrict__ boxes, uin
 }
 
 // boxes: [6][chunks] (launch_chunk_boxes).  Q as for knn_search_team (thr: the
-// cap, a seed's bound or that of a search that gave up).  bound_first: the
-// k-th distance within the nearest chunk bounds the search before it starts;
-// without it a wide bound lets most points of a group into the buffer (5,000
-// queries of 5,000 points about one cluster, k = 7, unseeded, no cap: 96 ->
-// 68 us; 131,072 of 1,254 mixed: 308 -> 116 us).
+// cap, a seed's bound or that of a search that gave up).  bound_first: two
+// passes that keep nothing but each lane's nearest points, over the nearest
+// chunk and then over the others within the k-th of those, bound the search
+// before it starts; without it a wide bound lets most points of a group into
+// the buffer (131,072 queries of 1,254 mixed points, k = 7, unseeded: 332 us,
+// with the nearest chunk's bound alone 58, here 54, k = 16 556 / 153 / 91; 5,000 of
+// 5,000 about one cluster 96 / 68 / 55).
 template <int G, int KM, int RF>
 __device__ __forceinline__ void knn_chunks_team(TeamList<G, KM, RF>& L, const FlatQuery& Q, bool bound_first, uint32_t nB,
                                                 const float4* __restrict__ bpos, const float* __restrict__ boxes) {
@@ -49,11 +51,21 @@ __device__ __forceinline__ void knn_chunks_team(TeamList<G, KM, RF>& L, const Fl
         const float near2 = -L.max_of(-best);
         if (near2 > L.lim) return;  // no chunk in reach
         if (near2 < INFINITY) {
-            const uint32_t who = L.votes(best == near2);
-            at = (uint32_t)__shfl((int)at, (int)(L.first + (uint32_t)__ffs((int)who) - 1u), 64);
+            const auto who = L.votes(best == near2);
+            at = (uint32_t)__shfl((int)at, (int)L.first + __ffsll((unsigned long long)who) - 1, 64);
+            typename TeamList<G, KM, RF>::Two two;
             int M = 0;
             L.push_run(at * 64u, L.lane == 0 ? min(64u, nB - at * 64u) : 0u, M);
-            L.lim = fminf(L.lim, L.bound_of(M, Q.x, Q.y, Q.z, Q.self, rb));
+            L.nearest(two, M, Q.x, Q.y, Q.z, Q.self, rb);
+            L.lim = fminf(L.lim, L.kth(two));
+            for (uint32_t c0 = 0; c0 < chunks; c0 += G) {
+                const uint32_t c = c0 + L.lane;
+                const float d2 = c < chunks && c != at ? chunk_gap2(boxes, chunks, c, q) : INFINITY;
+                M = 0;
+                L.push_run(c * 64u, (c < chunks && c != at && d2 <= L.lim) ? min(64u, nB - c * 64u) : 0u, M);
+                if (M != 0) L.nearest(two, M, Q.x, Q.y, Q.z, Q.self, rb);
+            }
+            L.lim = fminf(L.lim, L.kth(two));
         }
     }
     for (uint32_t c0 = 0; c0 < chunks; c0 += G) {

@@ -26,10 +26,11 @@ __global__ __launch_bounds__(kBlock) void k_knn_team(uint32_t nA, const float4* 
         if (seed)
             thr = fminf(cap2, team_seed_bound(L, active, seed, nA, (active && row_map) ? row_map[s] : s, nB, val_map,
                                                  q.x, q.y, q.z, bpos));
+        const bool bound_first = thr == INFINITY;
         // As k_knn_binned: no candidate within the cap of B's bounding box.
         if (box && active && box_beyond(box, q.x, q.y, q.z, cap2)) thr = -1.f;
         const FlatQuery Q{q.x, q.y, q.z, thr, self ? s : UINT32_MAX, active};
-        knn_search_team(L, Q, g, nB, bpos, bstart);
+        knn_search_team<false>(L, Q, g, nB, bpos, bstart, bound_first);
     }
     if (active) L.store(nA, s, out_idx, out_dist);
 }

@@ -12,6 +12,8 @@
 // The keys (d2 bits, agent index), the candidate set and the exactness test
 // are those of the flat search, so the lists are the same.
 #pragma once
+#include <type_traits>
+
 #include "gs_knn_core.hpp"
 
 namespace gs {
@@ -25,7 +27,11 @@ constexpr uint32_t kTeamMaxK = 16;
 // 18.6; 131,072 38.1 / 35.3 / 44.7; 262,144 50.7 / 57.5 / 77.6.  k = 16,
 // 65,536 64.2 / 48.1 / 39.7; 131,072 75.7 / 63.6 / 61.9; 262,144 110 / 98.4 /
 // 103; 524,288 160 / 175 / 201.  Four lanes were slower than eight
-// throughout (k = 7: 24.2 us at 16,384, 60.3 at 262,144).
+// throughout (k = 7: 24.2 us at 16,384, 60.3 at 262,144).  Near the lines a
+// lane is ahead where the seed is as good as it gets, in a uniform flock at rest
+// (131,072, k = 1 13 / 20, k = 4 18 / 24, k = 7 28 / 27; 262,144, k = 16 57 / 62),
+// and far behind in clumps (131,072, k = 7 102 / 59) or apart from its targets
+// (100,000 of 20,000, no cap 5,140 / 525, about one cluster 10,900 / 486).
 constexpr uint32_t kTeam16Max = 24576, kTeam8Max = 131072;          // k <= 8
 constexpr uint32_t kTeam16MaxLong = 131072, kTeam8MaxLong = 262144;  // longer lists
 inline int team_lanes(uint32_t n, uint32_t k) {
@@ -88,12 +94,22 @@ template <int G, int KM, int RF> struct TeamList {
         lim = INFINITY;
     }
     // Which lanes of the team hold p (bit = lane of the team).
-    __device__ __forceinline__ uint32_t votes(bool p) const {
-        return (uint32_t)(__ballot(p) >> first) & ((1u << G) - 1u);
+    typedef typename std::conditional<(G > 32), uint64_t, uint32_t>::type Mask;
+    __device__ __forceinline__ Mask votes(bool p) const {
+        return (Mask)(__ballot(p) >> first) & ((Mask)~(Mask)0 >> (8 * sizeof(Mask) - G));
     }
+    __device__ __forceinline__ static int count(Mask m) { return G > 32 ? __popcll(m) : __popc((uint32_t)m); }
+    // The lanes of the mask below this one.
+    __device__ __forceinline__ int rank(Mask m) const { return count(m & (((Mask)1 << lane) - 1)); }
     __device__ __forceinline__ float max_of(float v) const {
 #pragma unroll
         for (int off = G / 2; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+        return v;
+    }
+
+    __device__ __forceinline__ uint32_t sum_of(uint32_t v) const {
+#pragma unroll
+        for (int off = G / 2; off >= 1; off >>= 1) v += (uint32_t)__shfl_xor((int)v, off, 64);
         return v;
     }
 
@@ -130,9 +146,9 @@ template <int G, int KM, int RF> struct TeamList {
 
     // Appends each lane's run (len 0: none) to the M runs of the team.
     __device__ __forceinline__ void push_run(uint32_t t0, uint32_t len, int& M) {
-        const uint32_t m = votes(len != 0u);
-        if (len != 0u) run[M + __popc(m & ((1u << lane) - 1u))] = make_uint2(t0, len);
-        M += __popc(m);
+        const Mask m = votes(len != 0u);
+        if (len != 0u) run[M + rank(m)] = make_uint2(t0, len);
+        M += count(m);
     }
 
     // Walks the team's M runs in chunks of G slots, four chunks in flight:
@@ -177,18 +193,17 @@ template <int G, int KM, int RF> struct TeamList {
 #pragma unroll
             for (int h = 0; h < 4; h += 2) {
                 const bool pa = ok[h] && d2[h] <= lim, pb = ok[h + 1] && d2[h + 1] <= lim;
-                const uint32_t va = votes(pa), vb = votes(pb);
-                if ((va | vb) == 0u) continue;
-                const int na = __popc(va), total = na + __popc(vb);
+                const Mask va = votes(pa), vb = votes(pb);
+                if ((va | vb) == 0) continue;
+                const int na = count(va), total = na + count(vb);
                 if (cnt + total > Lds::cap) reduce();  // leaves at most k: the two chunks now fit
-                const uint32_t below = (1u << lane) - 1u;
                 if (pa) {
-                    const int at = cnt + __popc(va & below);
+                    const int at = cnt + rank(va);
                     key[at] = make_key(d2[h], id_of(p[h]));
                     slot[at] = t[h];
                 }
                 if (pb) {
-                    const int at = cnt + na + __popc(vb & below);
+                    const int at = cnt + na + rank(vb);
                     key[at] = make_key(d2[h + 1], id_of(p[h + 1]));
                     slot[at] = t[h + 1];
                 }
@@ -199,15 +214,15 @@ template <int G, int KM, int RF> struct TeamList {
 
     // Each lane's candidate, when it has one (pass).
     __device__ __forceinline__ void add(bool pass, float d2, uint32_t id, uint32_t t) {
-        const uint32_t v = votes(pass);
-        if (v == 0u) return;
-        if (cnt + __popc(v) > Lds::cap) reduce();
+        const Mask v = votes(pass);
+        if (v == 0) return;
+        if (cnt + count(v) > Lds::cap) reduce();
         if (pass) {
-            const int at = cnt + __popc(v & ((1u << lane) - 1u));
+            const int at = cnt + rank(v);
             key[at] = make_key(d2, id);
             slot[at] = t;
         }
-        cnt += __popc(v);
+        cnt += count(v);
     }
 
     // The sorted list to column `row` of the slot-major [k][n] output (pads
@@ -222,33 +237,47 @@ template <int G, int KM, int RF> struct TeamList {
         }
     }
 
-    // A bound on the k-th distance from the M runs: each lane's two nearest
-    // candidates are 2 G distinct points, and the k-th nearest of them lies
-    // no nearer than the k-th of all (+inf with fewer than k).
-    __device__ __forceinline__ float bound_of(int M, float qx, float qy, float qz, uint32_t self,
-                                              __amdgpu_buffer_rsrc_t rb) {
+    // A bound on the k-th distance: the lanes' two nearest candidates are
+    // distinct points, and the k-th nearest of them lies no nearer than the
+    // k-th of all (+inf with fewer than k).  Keeps nothing in LDS, so a
+    // pass over the runs costs little more than their loads.
+    struct Two {
         float a = INFINITY, b = INFINITY;
+    };
+    __device__ __forceinline__ void nearest(Two& two, int M, float qx, float qy, float qz, uint32_t self,
+                                            __amdgpu_buffer_rsrc_t rb) {
         walk(M, qx, qy, qz, self, rb, [&](const float* d2, const bool* ok, const uint32_t*, const float4*) {
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const float d = ok[u] && d2[u] < INFINITY ? d2[u] : INFINITY;  // a NaN is no candidate
-                b = fminf(b, fmaxf(a, d));
-                a = fminf(a, d);
+                two.b = fminf(two.b, fmaxf(two.a, d));
+                two.a = fminf(two.a, d);
             }
         });
-        float* v = (float*)key;
-        v[lane] = a;
-        v[G + lane] = b;
+    }
+    // The values are made distinct by their place in the low bits and ranked by
+    // counting; the bound has those bits set, a relative 2^-16 at most above.
+    __device__ __forceinline__ float kth(const Two& two) {
+        constexpr uint32_t N = G > 16 ? G : 2 * G;  // wide teams: the nearest of each lane
+        static_assert(KM <= (int)N && KM + (int)N / 2 <= Lds::cap, "the bound needs k values, and room for them");
+        uint32_t* v = (uint32_t*)(key + cnt);  // past the collected keys (fewer than k)
+        const uint32_t ua = (__float_as_uint(two.a) & ~(N - 1u)) | lane;
+        const uint32_t ub = (__float_as_uint(two.b) & ~(N - 1u)) | (G + lane);
+        v[lane] = ua;
+        if (N > G) v[G + lane] = ub;
         team_fence();
-        uint32_t ra = 0, rb2 = 0;
-#pragma unroll 4
-        for (uint32_t j = 0; j < 2u * G; ++j) {
-            const float o = v[j];
-            ra += (o < a || (o == a && j < lane)) ? 1u : 0u;
-            rb2 += (o < b || (o == b && j < G + lane)) ? 1u : 0u;
+        uint32_t ra = 0, rb = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < N / 2; ++j) {
+            const uint2 o = ((const uint2*)v)[j];
+            ra += (o.x < ua ? 1u : 0u) + (o.y < ua ? 1u : 0u);
+            if (N > G) rb += (o.x < ub ? 1u : 0u) + (o.y < ub ? 1u : 0u);
         }
         team_fence();
-        return max_of(ra == k - 1u ? a : (rb2 == k - 1u ? b : -1.f));
+        uint32_t u = 0u;
+        if (ra == k - 1u) u = ua | (N - 1u);
+        if (N > G && rb == k - 1u) u = ub | (N - 1u);
+        return max_of(u < 0x7F800000u ? __uint_as_float(u) : INFINITY);
     }
 };
 
@@ -281,13 +310,19 @@ __device__ __forceinline__ float team_seed_bound(const TeamList<G, KM, RF>& L, b
 // knn_search_flat; 1 <= nB < kFlatMaxPoints, k <= KM); RF is the first
 // box's column radius (1: 3 x 3, 2: 5 x 5 for lattices finer than the
 // neighbour distance).  Leaves the sorted list in L.  Called by every lane of
-// the wavefront; teams without a query pass active = false.  False when the
-// next box would have more than max_columns columns: L.lim is then a bound on
-// the k-th d2 (at most Q.thr) and the list is to be found another way.
-template <int G, int KM, int RF>
+// the wavefront; teams without a query pass active = false.  bound_first: the
+// box is walked twice, for a bound, then for the candidates within it.
+//
+// Local: false when the next box would have more columns than max_columns or more
+// cells than there are points, or when a ring's runs hold more than
+// kLocalCandidates; L.lim is then a bound on the k-th d2 (at most Q.thr) and the
+// list is to be found another way.
+constexpr uint32_t kLocalCandidates = 256;
+template <bool Local, int G, int KM, int RF>
 __device__ __forceinline__ bool knn_search_team(TeamList<G, KM, RF>& L, const FlatQuery& Q, const GridDev& g,
                                                 uint32_t nB, const float4* __restrict__ bpos,
-                                                const uint32_t* __restrict__ bstart, int max_columns = INT_MAX) {
+                                                const uint32_t* __restrict__ bstart, bool bound_first,
+                                                int max_columns = 0) {
     const __amdgpu_buffer_rsrc_t rb = pos_rsrc(bpos, nB);
     const float grow = 1.0f + 2e-5f;
     const float qx = Q.x, qy = Q.y, qz = Q.z;
@@ -302,9 +337,7 @@ __device__ __forceinline__ bool knn_search_team(TeamList<G, KM, RF>& L, const Fl
     // outside the box before (ring Rin) is one run, the others the two runs
     // above and below it.
     int R = RF, Rin = RF, M = 0;
-    // Without a seed or a cap the box is walked twice: for a bound, then for
-    // the candidates within it.
-    for (bool bound_first = L.lim == INFINITY && L.k <= 2u * G;; bound_first = false) {
+    for (;; bound_first = false) {
         constexpr int W = 2 * RF + 1, rounds = (W * W + G - 1) / G;
         const float bound = L.lim * grow;
         const int zlo = max(cz - RF * g.zr, 0), zhi = min(cz + RF * g.zr, g.dz - 1);
@@ -323,7 +356,9 @@ __device__ __forceinline__ bool knn_search_team(TeamList<G, KM, RF>& L, const Fl
 #pragma unroll
         for (int i = 0; i < rounds; ++i) L.push_run(r[i].x, r[i].y - r[i].x, M);
         if (!bound_first) break;
-        L.lim = L.bound_of(M, qx, qy, qz, Q.self, rb);
+        typename TeamList<G, KM, RF>::Two two;
+        L.nearest(two, M, qx, qy, qz, Q.self, rb);
+        L.lim = fminf(L.lim, L.kth(two));
     }
     int c0 = 0, columns = 0;
     bool last = false;  // nothing is left to scan after the runs at hand
@@ -352,6 +387,7 @@ __device__ __forceinline__ bool knn_search_team(TeamList<G, KM, RF>& L, const Fl
             }
             const uint32_t tlo = bstart[0], thi = bstart[(uint32_t)g.dx * (uint32_t)g.dy * (uint32_t)g.dz];
             if (box_beyond_points(g, R, thi - tlo)) {
+                if (Local) return false;
                 // More cells than points: every point again, the list's own
                 // among them (they lie within the bound).
                 L.cnt = 0;
@@ -360,7 +396,7 @@ __device__ __forceinline__ bool knn_search_team(TeamList<G, KM, RF>& L, const Fl
                 continue;
             }
             columns = (min(cx + R, g.dx - 1) - max(cx - R, 0) + 1) * (min(cy + R, g.dy - 1) - max(cy - R, 0) + 1);
-            if (columns > max_columns) return false;
+            if (Local && columns > max_columns) return false;
             c0 = 0;
         }
         const int Z = R * g.zr, Zin = Rin * g.zr;
@@ -379,6 +415,7 @@ __device__ __forceinline__ bool knn_search_team(TeamList<G, KM, RF>& L, const Fl
                                              min(edge ? cz + Z : cz - Zin - 1, g.dz - 1), base, g, bstart);
             const uint2 hi = flat_column_run(valid && !edge, gxy, bound, grow, qz, max(cz + Zin + 1, 0),
                                              min(cz + Z, g.dz - 1), base, g, bstart);
+            if (Local && L.sum_of((lo.y - lo.x) + (hi.y - hi.x)) > kLocalCandidates) return false;
             L.push_run(lo.x, lo.y - lo.x, M);
             L.push_run(hi.x, hi.y - hi.x, M);
         }

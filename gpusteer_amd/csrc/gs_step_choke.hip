@@ -54,10 +54,11 @@ __global__ __launch_bounds__(kBlock) void k_pair_search(PairSearch P) {
         if (l.seed)
             thr = fminf(thr, team_seed_bound(L, active, l.seed, nA, (active && l.row_map) ? l.row_map[s] : s, l.nB,
                                              l.val_map, q.x, q.y, q.z, l.bpos));
+        const bool bound_first = thr == INFINITY;
         if (l.box && active && box_beyond(l.box, q.x, q.y, q.z, l.cap2)) thr = -1.f;
         const FlatQuery Q{q.x, q.y, q.z, thr, l.self ? s : UINT32_MAX, active};
-        if (l.start) knn_search_team(L, Q, P.g, l.nB, l.bpos, l.start);
-        else knn_chunks_team(L, Q, thr == INFINITY, l.nB, l.bpos, l.boxes);
+        if (l.start) knn_search_team<false>(L, Q, P.g, l.nB, l.bpos, l.start, bound_first);
+        else knn_chunks_team(L, Q, bound_first, l.nB, l.bpos, l.boxes);
     }
     if (active) L.store(nA, s, l.idx, l.dist);
 }

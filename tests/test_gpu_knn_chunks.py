@@ -61,7 +61,10 @@ def _check(gs, ctx, orc, a, b, k, cells, cap):
     (256, 0, 8, (16, 1, 16), None), (3000, 2, 3, (40, 1, 40), None), (3000, 63, 3, (40, 1, 40), 25.0),
     (24576, 64, 4, (40, 1, 40), None), (24577, 65, 9, (40, 1, 40), None), (140000, 256, 3, (40, 1, 40), 50.0),
     (5000, 1254, 3, (512, 1, 512), 140.0), (30000, 1254, 16, (512, 1, 512), 140.0), (5000, 4096, 7, (512, 1, 512), None),
-    (5000, 5000, 7, (64, 1, 64), 62.0), (2000, 16384, 16, (64, 1, 64), None), (300, 10000, 1, (64, 1, 64), 200.0)])
+    (5000, 5000, 7, (64, 1, 64), 62.0), (2000, 16384, 16, (64, 1, 64), None), (300, 10000, 1, (64, 1, 64), 200.0),
+    (4096, 256, 7, (65, 1, 64), None), (4096, 257, 7, (65, 1, 64), None), (4097, 257, 7, (65, 1, 64), 60.0),
+    (4096, 5000, 16, (64, 1, 64), None), (1000, 16384, 7, (100, 1, 100), None), (1000, 16384, 8, (100, 1, 100), 30.0),
+    (140000, 1254, 16, (512, 1, 512), 140.0)])
 def test_lists(gs, ctx, orc, na, nb, k, cells, cap):
     print(f"case na={na} nb={nb} k={k} cells={cells} cap={cap}", flush=True)
     _check(gs, ctx, orc, _points(na, na), _points(nb, nb + 1) if nb else None, k, cells, cap)
@@ -72,7 +75,8 @@ def test_lists(gs, ctx, orc, na, nb, k, cells, cap):
 @pytest.mark.parametrize("where", ["mixed", "apart", "one cluster"])
 @pytest.mark.parametrize("na,nb,k,radius,cap", [
     (2000, 1025, 1, 1, 40.0), (2000, 1025, 7, 2, 75.0), (1999, 4096, 8, 1, None), (513, 1024, 9, 2, 1e6),
-    (300, 10000, 16, 1, 60.0), (16384, 257, 7, 1, None)])
+    (300, 10000, 16, 1, 60.0), (16384, 257, 7, 1, None), (8192, 3000, 7, 1, None), (8193, 3000, 16, 1, 1e6),
+    (500, 16000, 7, 2, 150.0)])
 def test_small_groups(gs, ctx, orc, where, na, nb, k, radius, cap):
     print(f"case {where} na={na} nb={nb} k={k} radius={radius} cap={cap}", flush=True)
     g = np.random.default_rng(na + nb)
@@ -99,6 +103,23 @@ def test_small_groups(gs, ctx, orc, where, na, nb, k, radius, cap):
         if step == 1:  # part of each group goes to the opposite face: seeds far away
             for G in (A, B):
                 gs.wrapWorld(G, worldSize=(150.0, 150.0, 150.0))
+    for h in (knn, bins, A, B):
+        h.close()
+
+
+# Every point in one place: the bounds of all lanes and chunks are equal.
+@pytest.mark.parametrize("na,nb,k,cells", [(300, 100, 7, (4, 1, 4)), (2000, 3000, 16, (16, 1, 16)),
+                                           (9000, 3000, 7, (16, 4, 16)), (30000, 1000, 3, (200, 1, 200))])
+def test_ties(gs, ctx, na, nb, k, cells):
+    bins = gs.KNNBinData(ctx, cells, SIZE)
+    A, B = _group(gs, ctx, _points(na, 8)), _group(gs, ctx, np.tile(np.float32([[7.0, 0.0, -11.0]]), (nb, 1)))
+    knn = gs.KNNData(ctx, na, k)
+    for G in (A, B):
+        gs.updateKNNDatabase(G, bins)
+    for _ in range(2):
+        gs.findKNearestNeighbors(A, knn, bins, B, 1)
+        idx, _ = knn.download()
+        np.testing.assert_array_equal(idx, np.tile(np.arange(k, dtype=np.uint32)[:, None], (1, na)))
     for h in (knn, bins, A, B):
         h.close()
 
