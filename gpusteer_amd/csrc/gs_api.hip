@@ -1298,6 +1298,26 @@ static uint64_t points_in_reach(const gs_group_s* B, const GridDev& g, uint32_t 
 // 71, all 54 / 332).
 constexpr uint64_t kWideCapPoints = 64;
 
+// Whether the exhaustive search of few targets by many queries goes by a lane
+// per query (k_knn_snap_brute) instead of a team: a lane's time is that of the
+// targets, one after the other, until its queries fill the chip, a team's that
+// of its queries.  Lane / team, us, k = 7: 32,768 queries 9 / 6 at 16 targets;
+// 65,536 9 / 10 at 16, 13 / 10 at 32; 131,072 6 / 14 at 4, 15 / 14 at 32, 22 / 17 at
+// 64; 1,048,576 17 / 79 at 1, 78 / 96 at 64, 117 / 105 at 128; k = 16, 1,048,576
+// 144 / 138 at 48.  Without a seed a team reads more: 65,536 13 / 15 at 32,
+// 131,072 22 / 39 at 64, 36 / 31 at 128, 1,048,576 175 / 206 at 256.  A lane skips
+// what its wavefront cannot reach, so that for very many queries the targets in
+// reach count: 1,048,576 queries of 1,254, 14 in reach 108 / 168 us, 102 in reach
+// 163 / 171, without a seed 163 / 345; 262,144 50 / 46, 72 / 47, without a seed 72
+// / 95.
+static bool few_targets(uint32_t nA, uint32_t nB, uint64_t reach, uint32_t k, bool seeded) {
+    if (k > kChunkMaxK) return true;
+    uint32_t few = nA / 4096u;
+    if (seeded) few = std::min(few, k <= 8 ? 96u : 40u);
+    else if (nA >= 1u << 16) few = std::min(std::max(nA / 2048u, 64u), 256u);
+    return nB <= few || (nA >= (seeded ? 1u << 19 : 1u << 18) && reach <= few);
+}
+
 // A small query group searching another small group over a wide reach: one lane
 // per query would run as a few dozen wavefronts, each walking the cells around
 // a query that the other group may be far from.  Such searches take the cells
@@ -1334,7 +1354,7 @@ static void find_knn(gs_group A, gs_knn out, gs_bins bins, gs_group B, uint32_t 
         !split && !(flags & GS_KNN_BINNED) && prefer_exhaustive(B, bins->g, bins->cells, max_distance);
     const Seed sd = seed_for(out, A, B, flags);
     const uint64_t reach = points_in_reach(B, bins->g, bins->cells, max_distance);
-    if (exhaustive && out->k > kChunkMaxK) {
+    if (exhaustive && few_targets(A->n, B->n, reach, out->k, sd.seed != nullptr)) {
         launch_knn_snap_brute(A, out, B, cap2);
     } else if ((split || exhaustive) && out->k <= kChunkMaxK && B->n <= kChunkMax) {
         // The cells around a query hold nothing of a sparse B.

@@ -502,7 +502,7 @@ bool launch_knn_team(gs_group_s* A, gs_knn_s* out, gs_group_s* B, uint32_t searc
                      const uint32_t* seed, const uint32_t* row_map, const uint32_t* val_map, bool dist);
 void launch_knn_brute(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2);
 // The binned search's semantics (position snapshots of both builds) by an
-// exhaustive scan, for small B.
+// exhaustive scan with one lane per query, for small B.
 void launch_knn_snap_brute(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2);
 constexpr uint32_t kSmallTargetSet = 256;
 // A sparse target set (fewer than one point per kSparseCells cells, at most

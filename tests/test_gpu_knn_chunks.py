@@ -107,6 +107,18 @@ def test_small_groups(gs, ctx, orc, where, na, nb, k, radius, cap):
         h.close()
 
 
+# Few targets of many queries, on both sides of the lines where a lane per query
+# takes over: with a seed and without, by the targets and by those in reach.
+@pytest.mark.parametrize("na,nb,k,cells,cap", [
+    (4096, 1, 3, (40, 1, 40), None), (65536, 16, 7, (40, 1, 40), None), (65536, 17, 16, (40, 1, 40), 50.0),
+    (65536, 64, 3, (40, 1, 40), None), (65535, 64, 3, (40, 1, 40), None), (131072, 33, 9, (40, 1, 40), None),
+    (262144, 128, 7, (64, 1, 64), None), (262144, 129, 16, (64, 1, 64), None),
+    (262144, 1254, 7, (512, 1, 512), 30.0), (524288, 1254, 3, (512, 1, 512), 12.0)])
+def test_few_targets(gs, ctx, orc, na, nb, k, cells, cap):
+    print(f"case na={na} nb={nb} k={k} cells={cells} cap={cap}", flush=True)
+    _check(gs, ctx, orc, _points(na, na), _points(nb, nb + 1), k, cells, cap)
+
+
 # Every point in one place: the bounds of all lanes and chunks are equal.
 @pytest.mark.parametrize("na,nb,k,cells", [(300, 100, 7, (4, 1, 4)), (2000, 3000, 16, (16, 1, 16)),
                                            (9000, 3000, 7, (16, 4, 16)), (30000, 1000, 3, (200, 1, 200))])
