@@ -231,6 +231,7 @@ _SIGS = {
     "gs_last_error": (C.c_char_p, []),
     "gs_version": (C.c_int, []),
     "gs_debug_fail_alloc_after": (C.c_int, [C.c_int64]),
+    "gs_debug_joint_frames": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint64)]),
     "gs_context_create": (C.c_int, [C.c_int, C.c_void_p, C.POINTER(_h)]),
     "gs_context_destroy": (C.c_int, [_h]),
     "gs_context_synchronize": (C.c_int, [_h]),

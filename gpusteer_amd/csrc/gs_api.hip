@@ -589,6 +589,15 @@ int gs_debug_fail_alloc_after(int64_t n) {
     return GS_OK;
 }
 
+/* Test hook: crowd frames of gs_step_choke issued jointly for both groups. */
+int gs_debug_joint_frames(gs_context ctx, uint64_t* n) {
+    return guarded([&] {
+        check(ctx, "context");
+        if (!n) fail(GS_ERR_INVALID_ARGUMENT, "out is NULL");
+        *n = ctx->joint_frames;
+    });
+}
+
 // ---- context -----------------------------------------------------------------
 int gs_context_create(int device, void* hip_stream, gs_context* out) {
     return guarded([&] {
@@ -1688,8 +1697,8 @@ static bool boids_step_once(gs_group_s* A, gs_knn_s* knn, gs_bins_s* bins, const
 // phase is bound by its launch and its latency), and every list is short and
 // its own container.
 static bool pair_frame_ok(gs_group_s* const A[2], const gs_group_s* W, const gs_group_s* O, const gs_bins_s* bins,
-                          gs_knn_s* const* knn, const gs_scenario* s, float cap) {
-    if (A[0] == A[1] || std::isnan(cap)) return false;
+                          gs_knn_s* const* knn) {
+    if (A[0] == A[1]) return false;
     const gs_context_s* ctx = A[0]->ctx;
     if (A[1]->ctx != ctx || W->ctx != ctx || O->ctx != ctx || bins->ctx != ctx) return false;
     for (int g = 0; g < 2; ++g)
@@ -1745,8 +1754,9 @@ int gs_step_choke(gs_group A0, gs_group A1, gs_group walls, gs_group obstacles, 
         const gs_flock_term& t = s->choke_separation;
         const float cap = s->other_max_distance > 0.f ? s->other_max_distance : INFINITY;
         for (uint32_t step = 0; step < steps; ++step) {
-            if (pair_frame_ok(A, walls, obstacles, bins, knn, s, cap)) {
+            if (pair_frame_ok(A, walls, obstacles, bins, knn)) {
                 pair_frame(A, walls, obstacles, bins, knn, s, cap2_of(cap));
+                ++A[0]->ctx->joint_frames;
                 continue;
             }
             ok(gs_update_knn_database(A[0], bins));

@@ -263,6 +263,7 @@ struct gs_context_s {
     bool own_stream = false;
     gs::LaunchShape shape[2];  // GS_SHAPE_KNN, GS_SHAPE_FLOCK
     gs::Staging stage;
+    uint64_t joint_frames = 0;  // gs_step_choke's, for tests
     uint32_t magic = 0x67736378u;
 };
 

@@ -1,8 +1,11 @@
 """Crowd frames phase by phase for both groups (gs_step_choke of small groups)
 against the separate calls: the whole state, storage order and every list."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from gpusteer_amd import _capi as capi
 from gpusteer_amd import scenarios
 from gpusteer_amd.ensemble import choke_step_calls, step_choke
 from gpusteer_amd.state import WallState
@@ -32,6 +35,12 @@ def _equal(a, b):
     for xs, ys in zip(a[1] + a[2], b[1] + b[2]):
         for x, y in zip(xs, ys):
             np.testing.assert_array_equal(x, y)
+
+
+def _joint_frames(ctx):
+    n = C.c_uint64()
+    capi.check(capi.lib.gs_debug_joint_frames(ctx.h, C.byref(n)), "gs_debug_joint_frames")
+    return n.value
 
 
 def _scenario(n0, n1, gap, mode, cells, obstacles=50, walls=True):
@@ -67,12 +76,15 @@ def test_equals_separate_calls(gs, ctx, n0, n1, k, mode, cells, obstacles, walls
     moved = any((st["px"] != r["px"]).any() for st, r in zip(sc.groups, want[0]))
     assert moved
     bins2, G2, W2, O2, knns2 = _world(gs, ctx, sc, k)
+    joint = 1 if max(n0, n1, bins.num_cells) <= 16384 else 0
+    before = _joint_frames(ctx)
     for parts in ((frames,), (1, 4, frames - 5)):
         for g, st in zip(G2, sc.groups):
             g.upload(st)
         for p in parts:
             step_choke(G2, knns2, W2, O2, bins2, sc, p)
         _equal(_result(G2, knns2, bins2.num_cells), want)
+    assert _joint_frames(ctx) - before == 2 * frames * joint
     # mixed with separate calls, and replayed from a recorded frame
     for g, st in zip(G2, sc.groups):
         g.upload(st)
