@@ -237,6 +237,40 @@ def test_calibration_workload_100_steps_vs_tangent(ctx, orc):
     assert _rel_ok(grad2, grad, 1e-4).all()
 
 
+# 98,304 agents are the most whose neighbours are searched by several lanes each.
+@pytest.mark.parametrize("crowds,n,k", [(4, 24576, 7), (8, 16384, 7), (8, 16384, 8)])
+def test_search_sizes(ctx, crowds, n, k):
+    """Together as one by one: states bit for bit, loss and gradient up to the
+    order of their sums in double precision (a power of two of crowds scales
+    every term exactly)."""
+    cfg = scenarios.CalibConfig(steps=4, checkpoint_every=2)
+    specs = scenarios.calib_scenarios(crowds, n)
+    for _, sc in specs:
+        sc.groups[1].arrays["pz"] += np.float32(40.0)  # the groups overlap
+    th = scenarios.calib_params()
+    ens = Ensemble(ctx, specs, k=k)
+    cal = Calibration(ens, cfg)
+    loss, grad = cal.forward(th), cal.backward()
+    one_loss, one_grad = 0.0, np.zeros(14)
+    for i, spec in enumerate(specs):
+        e = Ensemble(ctx, [spec], k=k)
+        c = Calibration(e, cfg)
+        one_loss += c.forward(th) / crowds
+        one_grad += c.backward() / crowds
+        for g in range(2):
+            a, b = cal.final_state(i, g), c.final_state(0, g)
+            for f in a.arrays:
+                np.testing.assert_array_equal(a.arrays[f], b.arrays[f], err_msg=f"scenario {i} group {g} field {f}")
+        c.close()
+        e.close()
+    cal.close()
+    ens.close()
+    # Sums of at most 4 steps x 1.3e5 terms: 5.2e5 x 2^-53 = 6e-11 of the sum of their
+    # magnitudes, which is the loss itself and less than 1,000 times a gradient.
+    assert abs(loss - one_loss) <= 6e-11 * abs(one_loss)
+    assert (np.abs(grad - one_grad) <= 6e-8 * np.max(np.abs(one_grad))).all(), (grad, one_grad)
+
+
 @pytest.mark.parametrize("n,k", [(200, 1), (200, 8), (10, 7), (12, 8)])
 def test_list_lengths(ctx, orc, n, k):
     """The shortest and longest lists, and groups with fewer neighbours than

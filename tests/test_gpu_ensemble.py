@@ -38,6 +38,33 @@ def test_ensemble_equals_sequential(ctx, mode):
     seq.close()
 
 
+# Beyond 24,576 agents (8 lanes per query), beyond 131,072 without crowds and
+# beyond 262,144 with them (one lane).
+@pytest.mark.parametrize("k,flocks,crowds", [(7, (9000, 11000), (3000, 7000)), (8, (20000,), (10000, 24000)),
+                                             (8, (66000, 66100), ()), (4, (2000,), (66000,) * 4),
+                                             (7, (2000,), (66000,) * 4)])
+def test_ensemble_search_sizes(ctx, k, flocks, crowds):
+    print(f"case k={k} flocks={flocks} crowds={crowds}", flush=True)
+    specs = []
+    for i, n in enumerate(flocks):
+        st, p = scenarios.boids_sphere(n=n, workload=60 + i)
+        p.grid_cells = (scenarios.boids_cells_for(n),) * 3
+        specs.append(("boids", st, p))
+    for i, n in enumerate(crowds):
+        sc = scenarios.choke(n_total=n, gap=10.0, workload=70 + i)
+        sc.groups[1].arrays["pz"] += np.float32(40.0)  # the groups overlap
+        c = scenarios.choke_cells_for(n)
+        sc.grid_cells = (c, 1, c)
+        specs.insert(2 * i + 1, ("choke", sc))
+    ens = Ensemble(ctx, specs, k=k)
+    seq = Sequential(ctx, specs, k=k)
+    ens.step(5)
+    seq.step(5)
+    _compare(ens, seq, specs, f"k={k}")
+    ens.close()
+    seq.close()
+
+
 def test_ensemble_graph_equals_eager(ctx):
     specs = scenarios.ensemble_mix(n_scenarios=4, n_min=500, n_max=2000, workload=12)
     a, b = Ensemble(ctx, specs), Ensemble(ctx, specs)

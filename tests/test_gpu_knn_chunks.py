@@ -71,12 +71,13 @@ def test_lists(gs, ctx, orc, na, nb, k, cells, cap):
 
 
 # Small groups by small groups: the cells around the query, wider boxes while
-# they have no more columns than the target has chunks, then the chunks.
+# they have no more columns than the target has chunks, then the chunks; the
+# split scan for more than 16 neighbours.
 @pytest.mark.parametrize("where", ["mixed", "apart", "one cluster"])
 @pytest.mark.parametrize("na,nb,k,radius,cap", [
     (2000, 1025, 1, 1, 40.0), (2000, 1025, 7, 2, 75.0), (1999, 4096, 8, 1, None), (513, 1024, 9, 2, 1e6),
     (300, 10000, 16, 1, 60.0), (16384, 257, 7, 1, None), (8192, 3000, 7, 1, None), (8193, 3000, 16, 1, 1e6),
-    (500, 16000, 7, 2, 150.0)])
+    (500, 16000, 7, 2, 150.0), (2000, 1025, 20, 1, 75.0), (1999, 4096, 32, 2, None), (513, 1024, 17, 1, 1e6)])
 def test_small_groups(gs, ctx, orc, where, na, nb, k, radius, cap):
     print(f"case {where} na={na} nb={nb} k={k} radius={radius} cap={cap}", flush=True)
     g = np.random.default_rng(na + nb)

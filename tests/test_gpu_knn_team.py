@@ -1,5 +1,5 @@
 """The several-lanes-per-query search at the sizes where its dispatch, its
-teams and its buffers have edges, bit-exact against the oracle's brute force
+teams and its buffers have edges (and the one-lane search beyond them), bit-exact against the oracle's brute force
 (on a sample of queries) and against the one-lane search (which a launch shape
 set on the context selects for k = 7)."""
 import numpy as np
@@ -61,7 +61,9 @@ def _search(gs, ctx, a, b, k, cells, radius=1, cap=None, calls=1):
     (1000, 7, (1, 1, 1), 1), (1000, 16, (30, 30, 30), 2), (2049, 9, (9, 7, 21), 1), (5000, 8, (30, 30, 60), 2),
     (5000, 7, (40, 1, 40), 1), (24576, 7, (20, 20, 20), 1), (24577, 7, (20, 20, 20), 1), (24577, 4, (50, 50, 50), 2),
     (131072, 7, (36, 36, 36), 1), (131073, 7, (36, 36, 36), 1), (131072, 16, (30, 30, 60), 1),
-    (131073, 16, (30, 30, 60), 1), (262144, 12, (40, 40, 80), 1), (262145, 12, (40, 40, 80), 1)])
+    (131073, 16, (30, 30, 60), 1), (262144, 12, (40, 40, 80), 1), (262145, 12, (40, 40, 80), 1),
+    (131073, 1, (36, 36, 36), 1), (131073, 4, (36, 36, 36), 1), (131073, 8, (30, 30, 90), 1), (131073, 5, (36, 36, 36), 2),
+    (131073, 8, (60, 1, 60), 1), (262145, 16, (40, 40, 80), 1), (262145, 9, (60, 60, 60), 2)])
 def test_lists_at_the_edges(gs, ctx, orc, n, k, cells, radius):
     print(f"case n={n} k={k} cells={cells} radius={radius}", flush=True)
     pos = _points(n, n + k, dims=2 if cells[1] == 1 and cells[0] > 1 else 3)
@@ -73,7 +75,9 @@ def test_lists_at_the_edges(gs, ctx, orc, n, k, cells, radius):
 
 
 @pytest.mark.parametrize("na,nb,k,cap", [(700, 3000, 7, 1.0), (3000, 700, 16, 2.5), (30000, 5000, 7, 0.5),
-                                         (300, 1, 7, 30.0), (5000, 5000, 3, 100.0)])
+                                         (300, 1, 7, 30.0), (5000, 5000, 3, 100.0),
+                                         (131073, 5000, 4, 1.0), (131073, 5000, 8, 2.5), (131073, 20000, 7, 0.5),
+                                         (262145, 5000, 16, 1.0), (262145, 5000, 9, 4.0)])
 def test_two_groups_within(gs, ctx, orc, na, nb, k, cap):
     a, b = _points(na, 1), _points(nb, 2)
     q = np.unique(np.linspace(0, na - 1, 300).astype(np.uint32))

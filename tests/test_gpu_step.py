@@ -415,3 +415,27 @@ def test_empty_group_steps(gs, ctx):
     assert E.download().n == 0
     for h in (E, bins, knn):
         h.close()
+
+
+@pytest.mark.parametrize("n,k,cells", [(131073, 4, (32, 32, 64)), (131073, 8, (32, 32, 64)), (262145, 13, (30, 30, 90))])
+def test_fused_steps_of_one_lane_searches(gs, ctx, orc, n, k, cells):
+    """Flocks just beyond the several-lanes-per-query search, with other lists
+    than the tuned ones: seeded steps equal the oracle's."""
+    print(f"case n={n} k={k} cells={cells}", flush=True)
+    size = 1000.0 * (n / float(1 << 20)) ** (1.0 / 3.0)
+    st, p = scenarios.boids_box(n=n, size=size, k=k)
+    p.grid_cells = cells
+    ref = st.copy()
+    A = gs.AgentGroup(ctx, st)
+    bins = gs.KNNBinData(ctx, p.grid_cells, p.grid_size, origin=p.grid_origin)
+    knn = gs.KNNData(ctx, n, k)
+    for steps in (1, 3):
+        gs.stepBoids(A, knn, bins, p, steps)
+        for _ in range(steps):
+            r_idx, r_dist = orc.boids_step(ref, p)
+        idx, dist = knn.download()
+        np.testing.assert_array_equal(idx, r_idx)
+        np.testing.assert_array_equal(dist, r_dist)
+        assert_state_equal(A.download(), ref, what=f"after {steps} more: ")
+    for h in (A, bins, knn):
+        h.close()
