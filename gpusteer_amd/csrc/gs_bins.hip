@@ -16,8 +16,9 @@
 //               every live field, the bits and the agent index are written
 //               there in the alternate buffers, with the old <-> new maps.
 // Because the previous build left the state in cell order and agents move
-// little between builds, the reorder's writes land nearly sequentially.  The counts array is all-zero between builds (pass 2 clears it),
-// so no memset is recorded in the stream.
+// little between builds, the reorder's writes land nearly sequentially.  The
+// counts array is all-zero between builds (pass 2 clears it), so no memset is
+// recorded in the stream.
 #include <algorithm>
 
 #include "gs_internal.hpp"

@@ -23,7 +23,8 @@
 
 namespace gs {
 
-template <int KMAX>
+constexpr int kSplitK = GS_MAX_K;  // longest list
+
 __global__ __launch_bounds__(kBlock) void k_knn_split_part(uint32_t nA, const float4* __restrict__ apos, uint32_t nB,
                                                            const float4* __restrict__ bpos, int self, uint32_t k,
                                                            float cap2, uint32_t chunk,
@@ -38,7 +39,7 @@ __global__ __launch_bounds__(kBlock) void k_knn_split_part(uint32_t nA, const fl
     const float4 q = active ? apos[s] : make_float4(0.f, 0.f, 0.f, 0.f);
     const uint32_t skip = (self && active) ? s : UINT32_MAX;
     const uint32_t b0 = blockIdx.y * chunk, b1 = min(b0 + chunk, nB);
-    TopK<KMAX> h;
+    TopK<kSplitK> h;
     h.init(k);
     // A candidate can enter only with d2 <= lim: the cap and, with a seed
     // (the container's previous exact result), the largest current d2 to
@@ -46,7 +47,7 @@ __global__ __launch_bounds__(kBlock) void k_knn_split_part(uint32_t nA, const fl
     // the list's own k-th d2.  Inactive lanes take none.
     float lim = -INFINITY;
     if (active)
-        lim = fminf(cap2, seed ? seed_bound<KMAX>(seed, k, nA, row_map ? row_map[s] : s, nB, val_map, q.x, q.y,
+        lim = fminf(cap2, seed ? seed_bound<kSplitK>(seed, k, nA, row_map ? row_map[s] : s, nB, val_map, q.x, q.y,
                                                   q.z, bpos)
                                : INFINITY);
     // The fused d2 filters against the widened limit; a passing candidate's
@@ -148,16 +149,15 @@ __global__ __launch_bounds__(kBlock) void k_knn_split_part(uint32_t nA, const fl
     // merge's lane reads its range's list as k consecutive entries.
     const size_t o0 = ((size_t)blockIdx.y * nA + s) * k;
 #pragma unroll
-    for (int j = 0; j < KMAX; ++j) {
-        if (j >= KMAX - (int)k) {
-            const size_t o = o0 + (uint32_t)(j - (KMAX - (int)k));
+    for (int j = 0; j < kSplitK; ++j) {
+        if (j >= kSplitK - (int)k) {
+            const size_t o = o0 + (uint32_t)(j - (kSplitK - (int)k));
             part_key[o] = h.key[j];
             part_slot[o] = h.t[j];
         }
     }
 }
 
-template <int KMAX>
 __global__ __launch_bounds__(kBlock) void k_knn_split_merge(uint32_t nA, uint32_t S, uint32_t k,
                                                             const uint64_t* __restrict__ part_key,
                                                             const uint32_t* __restrict__ part_slot,
@@ -166,10 +166,10 @@ __global__ __launch_bounds__(kBlock) void k_knn_split_merge(uint32_t nA, uint32_
     const uint32_t s = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
     if (s >= nA) return;  // the whole wavefront
-    uint64_t key[KMAX];
-    uint32_t t[KMAX];
+    uint64_t key[kSplitK];
+    uint32_t t[kSplitK];
 #pragma unroll
-    for (int j = 0; j < KMAX; ++j) {
+    for (int j = 0; j < kSplitK; ++j) {
         key[j] = kKeyEmpty;
         t[j] = UINT32_MAX;
         if (lane < S && (uint32_t)j < k) {
@@ -197,12 +197,12 @@ __global__ __launch_bounds__(kBlock) void k_knn_split_merge(uint32_t nA, uint32_
         }
         const bool adv = (int)lane == owner;
 #pragma unroll
-        for (int j = 0; j < KMAX - 1; ++j) {
+        for (int j = 0; j < kSplitK - 1; ++j) {
             key[j] = adv ? key[j + 1] : key[j];
             t[j] = adv ? t[j + 1] : t[j];
         }
-        key[KMAX - 1] = adv ? kKeyEmpty : key[KMAX - 1];
-        t[KMAX - 1] = adv ? UINT32_MAX : t[KMAX - 1];
+        key[kSplitK - 1] = adv ? kKeyEmpty : key[kSplitK - 1];
+        t[kSplitK - 1] = adv ? UINT32_MAX : t[kSplitK - 1];
     }
 }
 
@@ -214,7 +214,6 @@ uint32_t knn_split_ranges(uint32_t nA, uint32_t nB) {
     return S;
 }
 
-template <int KMAX>
 static void run_split(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, uint32_t S, const uint32_t* seed,
                       const uint32_t* row_map, const uint32_t* val_map) {
     const uint32_t nA = A->n, nB = B->n, k = out->k;
@@ -225,10 +224,10 @@ static void run_split(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, u
     out->part_slot.reserve(parts);
     hipStream_t st = A->ctx->stream;
     const dim3 grid(blocks_for(nA), S);
-    k_knn_split_part<KMAX><<<grid, kBlock, 0, st>>>(nA, A->spos.p, nB, B->spos.p, A == B ? 1 : 0, k, cap2, chunk,
+    k_knn_split_part<<<grid, kBlock, 0, st>>>(nA, A->spos.p, nB, B->spos.p, A == B ? 1 : 0, k, cap2, chunk,
                                                     seed, row_map, val_map, out->part_key.p, out->part_slot.p);
     GS_LAUNCHED("k_knn_split_part");
-    k_knn_split_merge<KMAX><<<(nA + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, st>>>(
+    k_knn_split_merge<<<(nA + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, st>>>(
         nA, S, k, out->part_key.p, out->part_slot.p, out->idx_alt(), out->dist_alt());
     GS_LAUNCHED("k_knn_split_merge");
 }
@@ -241,7 +240,7 @@ void launch_knn_split(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2, c
         launch_knn_snap_brute(A, out, B, cap2);
         return;
     }
-    run_split<32>(A, out, B, cap2, S, seed, row_map, val_map);
+    run_split(A, out, B, cap2, S, seed, row_map, val_map);
 }
 
 }  // namespace gs

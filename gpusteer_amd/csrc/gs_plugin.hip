@@ -385,12 +385,10 @@ void launch_avoid_neighbors(gs_group_s* A, gs_knn_s* knn, gs_group_s* B, float m
                             int avoid_close, float w, uint32_t mask, int mode) {
     if (A->n == 0) return;
     hipStream_t st = A->ctx->stream;
-#define GS_AN(M)                                                                                                  \
-    k_avoid_neighbors<M><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(                                        \
-        A->n, A->dev_agents(), B->n, B->F(0), B->F(1),                                                             \
-                                                              B->F(2), B->F(3), B->F(4), B->F(5), B->F(6),        \
-                                                              B->F(19), knn->idx(), knn->dist(), knn->k, min_time, \
-                                                              min_sep, avoid_close, w, mask)
+#define GS_AN(M)                                                                                                 \
+    k_avoid_neighbors<M><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(                                      \
+        A->n, A->dev_agents(), B->n, B->F(0), B->F(1), B->F(2), B->F(3), B->F(4), B->F(5), B->F(6), B->F(19),    \
+        knn->idx(), knn->dist(), knn->k, min_time, min_sep, avoid_close, w, mask)
     if (mode == GS_MODE_GPUREF) GS_AN(GS_MODE_GPUREF);
     else GS_AN(GS_MODE_OPENSTEER);
 #undef GS_AN
@@ -404,8 +402,7 @@ void launch_update_anti_penetration(gs_group_s* A, gs_knn_s* knn, gs_group_s* W,
     gs_walls wd{W->F(f0), W->F(f0 + 1), W->F(f0 + 2), W->F(f0 + 3), W->F(f0 + 4),
                 W->F(f0 + 5), W->F(f0 + 6), W->F(f0 + 7), W->F(f0 + 8)};
     k_update_anti_penetration<<<agent_blocks(A->n), agent_block(A->n), 0, A->ctx->stream>>>(
-        A->n, A->dev_agents(), W->n, wd,
-                                                                                knn->idx(), knn->k, dt, closest);
+        A->n, A->dev_agents(), W->n, wd, knn->idx(), knn->k, dt, closest);
     GS_LAUNCHED("k_update_anti_penetration");
     // kinematic fields rewritten, steering zeroed, bits kept (some set)
     A->mark_integrated();
@@ -430,8 +427,7 @@ void launch_follow_path(gs_group_s* A, const gs_path_s* p, float prediction_time
     const uint32_t m = p->m;
     PathDev P{d, d + m, d + 2 * m, d + 3 * m, d + 4 * m, d + 5 * m, d + 6 * m, m, p->radius, p->total, p->cyclic};
     k_follow_path<<<agent_blocks(A->n), agent_block(A->n), 0, A->ctx->stream>>>(
-        A->n, A->dev_agents(), P, prediction_time, w,
-                                                                    mask);
+        A->n, A->dev_agents(), P, prediction_time, w, mask);
     GS_LAUNCHED("k_follow_path");
     A->mark_written(kFSteer, true);
 }

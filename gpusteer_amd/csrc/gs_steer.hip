@@ -160,11 +160,10 @@ static void run_flock(gs_group_s* A, gs_knn_s* knn, gs_group_s* B, const gs_floc
                       const gs_flock_term* ali, const gs_flock_term* coh, int mode) {
     hipStream_t st = A->ctx->stream;
     const Agents a = A->dev_agents();
-#define GS_FLOCK(MODE)                                                                                              \
-    k_flock<KMAX, MODE><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(                                         \
-        A->n, a, B->n, B->F(0), B->F(1), B->F(2), B->F(3),                                                         \
-                                                             B->F(4), B->F(5), knn->idx(), knn->k, term(sep),        \
-                                                             term(ali), term(coh))
+#define GS_FLOCK(MODE)                                                                                         \
+    k_flock<KMAX, MODE><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(                                     \
+        A->n, a, B->n, B->F(0), B->F(1), B->F(2), B->F(3), B->F(4), B->F(5), knn->idx(), knn->k, term(sep),    \
+        term(ali), term(coh))
     if (mode == GS_MODE_GPUREF) GS_FLOCK(GS_MODE_GPUREF);
     else GS_FLOCK(GS_MODE_OPENSTEER);
 #undef GS_FLOCK
@@ -188,8 +187,7 @@ void launch_seek(gs_group_s* A, const float* t, float w, uint32_t mask, int mode
             A->n, A->dev_agents(), t[0], t[1], t[2], w, mask);
     else
         k_seek<GS_MODE_OPENSTEER><<<agent_blocks(A->n), agent_block(A->n), 0, st>>>(
-            A->n, A->dev_agents(), t[0], t[1], t[2], w,
-                                                                       mask);
+            A->n, A->dev_agents(), t[0], t[1], t[2], w, mask);
     GS_LAUNCHED("k_seek");
     A->mark_written(kFSteer, true);
 }
@@ -197,9 +195,7 @@ void launch_seek(gs_group_s* A, const float* t, float w, uint32_t mask, int mode
 void launch_avoid_obstacles(gs_group_s* A, gs_group_s* O, gs_knn_s* knn, float min_time, float w, uint32_t mask) {
     if (A->n == 0) return;
     k_avoid_obstacles<<<agent_blocks(A->n), agent_block(A->n), 0, A->ctx->stream>>>(
-        A->n, A->dev_agents(), O->n, O->F(0),
-                                                                        O->F(1), O->F(2), O->F(19), knn->idx(),
-                                                                        knn->k, min_time, w, mask);
+        A->n, A->dev_agents(), O->n, O->F(0), O->F(1), O->F(2), O->F(19), knn->idx(), knn->k, min_time, w, mask);
     GS_LAUNCHED("k_avoid_obstacles");
     A->mark_written(kFSteer, true);
 }
@@ -210,8 +206,7 @@ void launch_avoid_walls(gs_group_s* A, gs_knn_s* knn, gs_group_s* W, float min_t
     gs_walls wd{W->F(f0), W->F(f0 + 1), W->F(f0 + 2), W->F(f0 + 3), W->F(f0 + 4),
                 W->F(f0 + 5), W->F(f0 + 6), W->F(f0 + 7), W->F(f0 + 8)};
     k_avoid_walls<<<agent_blocks(A->n), agent_block(A->n), 0, A->ctx->stream>>>(
-        A->n, A->dev_agents(), W->n, wd, knn->idx(),
-                                                                    knn->k, min_time, w, mask);
+        A->n, A->dev_agents(), W->n, wd, knn->idx(), knn->k, min_time, w, mask);
     GS_LAUNCHED("k_avoid_walls");
     // touching agents are moved and turned (positions, forward vectors)
     A->mark_written(kFSteer | 0x3Fu, true);

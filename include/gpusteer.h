@@ -237,7 +237,8 @@ int gs_update_knn_database(gs_group g, gs_bins bins);
  * 16384 agents each, at most 2^26 pairs) over more than 64 cells of reach is
  * served by the cells around each query and then by B's snapshot in chunks
  * (k > 16: by a scan split over many wavefronts), and a small or sparse B by
- * its chunks alone: the same exact result. */
+ * its chunks alone (few targets of many queries, and k > 16: by one lane per
+ * query): the same exact result. */
 int gs_find_knn(gs_group A, gs_knn out, gs_bins bins, gs_group B, uint32_t search_radius, uint32_t flags);
 /* gs_find_knn restricted to points closer than max_distance (strict, the
  * locality test of src/lq.c:327: d^2 < r^2 in fp32); rows with fewer than k
@@ -346,10 +347,13 @@ int gs_clear_bits(gs_group A);
  * launch shape the caller may set per context: block_threads in {128, 256,
  * 512} threads per block and agents_per_lane in {1, 2} (a lane handles that
  * many agent slots, so a wavefront covers 64 x agents_per_lane agents).
- * Default 256 x 1; smaller groups are searched by several lanes per query
- * unless another search shape is set.  Results do not depend on the shape.  gpusteer_amd's
- * autotuner picks the shapes by timing them on the workload.  Other values
- * return GS_ERR_UNSUPPORTED.  No counterpart in the reference (fixed
+ * 256 x 1 is the default and leaves the library its own choice for smaller
+ * groups: several lanes per query in the search, blocks of 64 threads in the
+ * flocking kernel up to 32768 agents; the other shapes are taken at any size.
+ * (Searches of small or sparse targets and crowd frames of two small groups
+ * have launch shapes of their own.)  Results do not depend on the shape.
+ * gpusteer_amd's autotuner picks the shapes by timing them on the workload.
+ * Other values return GS_ERR_UNSUPPORTED.  No counterpart in the reference (fixed
  * block size THREADSPERBLOCK = 256, include/OpenSteer/CUDA/CUDAKernelGlobals.cuh:9). */
 enum { GS_SHAPE_KNN = 0, GS_SHAPE_FLOCK = 1 };
 int gs_context_set_shape(gs_context ctx, int kernel, uint32_t block_threads, uint32_t agents_per_lane);
