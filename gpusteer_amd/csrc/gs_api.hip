@@ -1304,8 +1304,9 @@ static uint64_t points_in_reach(const gs_group_s* B, const GridDev& g, uint32_t 
 // A search without a seed looks for a bound first when it reaches more points
 // than this: with fewer the bound costs more than it saves (131,072 queries of
 // 1,254 walls, k = 7, bound first / not: 14 in reach 49 / 28 us, 102 in reach 53 /
-// 71, all 54 / 332).
-constexpr uint64_t kWideCapPoints = 64;
+// 71, all 54 / 332; through the bins 20,000 of 20,000, 76 in reach 26 / 22,
+// 131,072 of 131,072, 500 in reach 47 / 94, k = 16 89 / 153).
+constexpr uint64_t kWideCapPoints = 96;
 
 // Whether the exhaustive search of few targets by many queries goes by a lane
 // per query (k_knn_snap_brute) instead of a team: a lane's time is that of the
@@ -1373,7 +1374,8 @@ static void find_knn(gs_group A, gs_knn out, gs_bins bins, gs_group B, uint32_t 
     } else if (split) {
         launch_knn_split(A, out, B, cap2, sd.seed, sd.row_map, sd.val_map);
     } else {
-        launch_knn_binned(A, out, B, search_radius, cap2, sd.seed, sd.row_map, sd.val_map);
+        launch_knn_binned(A, out, B, search_radius, cap2, sd.seed, sd.row_map, sd.val_map, true,
+                          reach > kWideCapPoints);
     }
     out->cur ^= 1;
     mark_result(out, A, B);

@@ -495,12 +495,15 @@ void launch_bins_build(gs_group_s* g, const gs_bins_s* b, int wrap_shape, const 
 // cap2: only points with d2 <= cap2 qualify (+inf: no cap).
 // dist false: the alternate distance buffer is left unwritten (a caller that
 // reads only the indices before the next search).
+// wide_cap: the cap is likely to hold many more points than a list.
 void launch_knn_binned(gs_group_s* A, gs_knn_s* out, gs_group_s* B, uint32_t search_radius, float cap2,
-                       const uint32_t* seed, const uint32_t* row_map, const uint32_t* val_map, bool dist = true);
+                       const uint32_t* seed, const uint32_t* row_map, const uint32_t* val_map, bool dist = true,
+                       bool wide_cap = false);
 // The same search by several lanes per query, where A's query count asks for
 // it (returns whether it did).
 bool launch_knn_team(gs_group_s* A, gs_knn_s* out, gs_group_s* B, uint32_t search_radius, float cap2,
-                     const uint32_t* seed, const uint32_t* row_map, const uint32_t* val_map, bool dist);
+                     const uint32_t* seed, const uint32_t* row_map, const uint32_t* val_map, bool dist,
+                     bool wide_cap);
 void launch_knn_brute(gs_group_s* A, gs_knn_s* out, gs_group_s* B, float cap2);
 // The binned search's semantics (position snapshots of both builds) by an
 // exhaustive scan with one lane per query, for small B.

@@ -76,6 +76,7 @@ def test_lists_at_the_edges(gs, ctx, orc, n, k, cells, radius):
 
 @pytest.mark.parametrize("na,nb,k,cap", [(700, 3000, 7, 1.0), (3000, 700, 16, 2.5), (30000, 5000, 7, 0.5),
                                          (300, 1, 7, 30.0), (5000, 5000, 3, 100.0),
+                                         (30000, 20000, 7, 6.0), (9000, 30000, 16, 4.0), (30000, 18000, 7, 1.9), (30000, 18000, 7, 2.1),
                                          (131073, 5000, 4, 1.0), (131073, 5000, 8, 2.5), (131073, 20000, 7, 0.5),
                                          (262145, 5000, 16, 1.0), (262145, 5000, 9, 4.0)])
 def test_two_groups_within(gs, ctx, orc, na, nb, k, cap):
