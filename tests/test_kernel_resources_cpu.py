@@ -76,6 +76,8 @@ BUDGETS = [
     (r"e_knnILi8ELi1E", 152, 0),
     (r"k_knn_teamILi", 96, 0),                       # several lanes per query: 5 wavefronts per SIMD
     (r"e_knn_teamILi", 96, 0),
+    (r"k_knn_chunksILi", 96, 0),
+    (r"k_pair_search", 96, 0),
     (r"k_knn_split_part", 400, 0),
     (r"k_knn_split_merge", 128, 0),
     (r"c4_backward", 128, 0),
